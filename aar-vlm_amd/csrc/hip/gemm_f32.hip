@@ -39,282 +39,12 @@
 
 #include "colsum.hpp"
 #include "common.hpp"
+#include "gemm_epi.hpp"
 #include "gemm_small.hpp"
+#include "gemm_split.hpp"
 
 namespace aar {
 namespace {
-
-constexpr int kGroupM = 4;
-
-__device__ __forceinline__ void map_tile(int tiles_m, int tiles_n, int& tm, int& tn) {
-  int w = blockIdx.x;
-  const int nb = gridDim.x;
-  if ((nb & 7) == 0) w = (w & 7) * (nb >> 3) + (w >> 3);  // XCD-contiguous ranges
-  const int group_size = kGroupM * tiles_n;
-  const int group = w / group_size;
-  const int first_m = group * kGroupM;
-  const int rows = min(tiles_m - first_m, kGroupM);
-  const int in_group = w - group * group_size;
-  tm = first_m + in_group % rows;
-  tn = in_group / rows;
-}
-
-// Epilogues (a template argument, because every one but the plain store
-// needs the accumulators in VGPRs: the kernels without one store straight
-// from the accumulators and keep their occupancy).  Each is the same fp32
-// operation as the separate op applied to the stored product:
-//   kEpiBias      C = acc + bias[col]            (linear layer: add_bias)
-//   kEpiBiasRelu  C = max(0, acc + bias[col])    (linear layer, then relu)
-//   kEpiMask      C = aux[row][col] > 0 ? acc : 0  (relu backward, aux = the
-//                 relu's output, which is positive exactly where its input is;
-//                 aux has C's layout)
-//   kEpiAdd       C = acc + aux[row][col]          (a residual add after the
-//                 product: x + y W^T)
-//   kEpiBiasAdd   C = (acc + bias[col]) + aux[row][col]  (the same after a
-//                 linear layer with a bias)
-// and two that carry a relu's mask as bits from the forward product to the
-// backward one (store_tile_bits), so the backward reads 1 bit per element
-// where kEpiMask reads the relu's whole output:
-//   kEpiBiasReluBits  C = max(0, acc + bias[col]) as kEpiBiasRelu, and bit
-//                     row % 32 of word bits[(row / 32) * N + col] set where
-//                     C > 0: a word holds one column of a 32-row block, the
-//                     rows of one accumulator block
-//   kEpiMaskBits      C = bit(row, col) ? acc : 0 (the relu backward), and
-//                     part[row / 64][col] = the sum of C over the 64 rows of
-//                     that chunk, in aar_colsum_f32's stage-1 order (two
-//                     running sums, see colsum_stage1_kernel): its partials
-//                     (a wave owns one chunk)
-enum : int {
-  kEpiNone = 0,
-  kEpiBias = 1,
-  kEpiBiasRelu = 2,
-  kEpiMask = 3,
-  kEpiAdd = 4,
-  kEpiBiasAdd = 5,
-  kEpiBiasReluBits = 6,
-  kEpiMaskBits = 7,
-  kEpiColsumA = 8
-};
-// kEpiColsumA is not an epilogue but work in the main loop (TN only): C is
-// stored plainly, and the waves of the first column of waves also sum the
-// staged A tile's columns: part[k / 64][m] = the sum of A[k][m] over the
-// 64-row chunk of k, in aar_colsum_f32's stage-1 order.  A lane holds the
-// k's with k & 4 == 4h of its column in order, i.e. one of that order's two
-// running sums; the halves add them at the chunk's end.  Chunk q is summed by
-// the workgroups with tn == q % tiles_n, so the work spreads over the grid.
-struct GemmEpi {
-  const float* bias;
-  const float* aux;
-  uint32_t* bits = nullptr;  // [ceil(M / 32)][N]: kEpiBiasReluBits writes, kEpiMaskBits reads
-  float* part = nullptr;     // kEpiMaskBits: [M / 64][N] column partials; kEpiColsumA: [K / 64][M]
-};
-constexpr bool epi_bits(int epi) { return epi == kEpiBiasReluBits || epi == kEpiMaskBits; }
-constexpr bool epi_dma_only(int epi) { return epi_bits(epi) || epi == kEpiColsumA; }
-
-// Epilogue: a wave's (32*TM) x (32*TN) accumulators to C.  Accumulator
-// layout of a 32x32 block: lane (lr, h), register r holds row
-// 8*(r/4) + 4*h + (r%4), column lr.
-// A wave tile wholly inside C (the common case) stores without bounds tests;
-// element offsets from the lane's first element are a constant row count
-// times ldc, which the compiler forms once in scalar registers.
-// NQ < 4: only register quads q0 .. q0 + NQ - 1 of each accumulator are
-// stored, their values held in quads 0 .. NQ - 1 of acc (a K group's share).
-constexpr bool epi_has_bias(int epi) {
-  return epi == kEpiBias || epi == kEpiBiasRelu || epi == kEpiBiasAdd || epi == kEpiBiasReluBits;
-}
-
-// The bias values a lane's accumulator columns need (column c0 + 32 j + lr),
-// read before the main loop so their latency is hidden under it: read at
-// the epilogue, they cost a memory round trip per workgroup round (measured
-// +10 us on a 16384 x 1536 x 384 product with the bias epilogue).
-template <int TN, int EPI>
-__device__ __forceinline__ void load_bias(const GemmEpi& ep, int64_t N, int64_t c0, int lr, float (&bias)[TN]) {
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int64_t col = c0 + 32 * j + lr;
-    bias[j] = 0.f;
-    if constexpr (epi_has_bias(EPI)) bias[j] = col < N ? ep.bias[col] : 0.f;
-  }
-}
-
-// Mask words the kEpiMaskBits epilogue needs, read before the main loop like
-// the bias: lane (lr, h) holds, for block (i, j), the word of column
-// c0 + 32 j + lr over rows r0 + 32 i .. + 31 (both halves read the same word,
-// 128 contiguous bytes per half-wave).
-template <int TM, int TN, int EPI>
-__device__ __forceinline__ void load_bits(const GemmEpi& ep, int64_t M, int64_t N, int64_t r0, int64_t c0, int lr,
-                                          uint32_t (&words)[TM][TN]) {
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      words[i][j] = 0u;
-      if constexpr (EPI == kEpiMaskBits) {
-        const int64_t col = c0 + 32 * j + lr;
-        if (r0 + 32 * i < M && col < N) words[i][j] = ep.bits[((r0 + 32 * i) >> 5) * N + col];
-      }
-    }
-}
-
-// The two mask-bit epilogues (see kEpiBiasReluBits / kEpiMaskBits).  Wave
-// tiles start at multiples of 32 rows, so accumulator block (i, j) covers
-// whole mask words: lane (lr, h) holds the bits 8 (r / 4) + 4 h + r % 4 of the
-// word of its column c0 + 32 j + lr, its half's 16 rows.
-//   kEpiBiasReluBits: each lane sets its 16 bits, the two halves OR their
-//   words (v_permlane32_swap) and half 0 stores the word.
-//   kEpiMaskBits (WM = 64: the wave's rows are one 64-row chunk): each lane
-//   tests its 16 bits of the prefetched word and sums its 32 rows of the
-//   chunk in order, the row set (row & 4 == 4h) of one of colsum's two
-//   running sums; half 0 adds its partner's (v_permlane32_swap) and stores
-//   the chunk partial s0 + s1.
-// The swap hands each lane its own value and its partner's, one in each
-// result; where the two are equal either is the partner's.
-__device__ __forceinline__ uint32_t partner_u32(uint32_t u) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return sw[0] == u ? sw[1] : sw[0];
-#else
-  return u;
-#endif
-}
-
-template <int TM, int TN, int EPI>
-__device__ __forceinline__ void store_tile_bits(const f32x16 (&acc)[TM][TN], float* __restrict__ C,
-                                                const GemmEpi& ep, const float (&bias)[TN],
-                                                const uint32_t (&words)[TM][TN], int64_t M, int64_t N, int64_t ldc,
-                                                int64_t r0, int64_t c0, int lr, int h) {
-  static_assert(epi_bits(EPI), "mask-bit epilogues only");
-  static_assert(EPI != kEpiMaskBits || TM == 2, "a kEpiMaskBits wave owns one 64-row chunk");
-  // addressing as store_tile: a lane base and row offsets dr * ldc that the
-  // compiler forms in scalar registers, bounds tests only off the interior
-  const bool interior = r0 + 32 * TM <= M && c0 + 32 * TN <= N;
-  float* const Cl = C + (r0 + 4 * h) * ldc + c0 + lr;
-  wait_vm_lgkm0<0>();  // bias / mask words (see store_tile)
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int64_t col = c0 + 32 * j + lr;
-    float vals[TM][16];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      uint32_t w = 0u;                           // this half's bits, at 8 (r / 4) + r % 4
-      const uint32_t mine = words[i][j] >> (4 * h);  // kEpiMaskBits: the same positions
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int dr = 32 * i + 8 * (r >> 2) + (r & 3);  // row - r0 - 4h
-        const int bit = 8 * (r >> 2) + (r & 3);
-        const bool ok = interior || (r0 + 4 * h + dr < M && col < N);
-        float v;
-        // (the bit tests stay free of the bounds test: with it, the compiler
-        // kept every element's lane mask live and spilled them to VGPR lanes)
-        if constexpr (EPI == kEpiBiasReluBits) {
-          v = fmaxf(0.0f, acc[i][j][r] + bias[j]);
-          w |= v > 0.0f ? (1u << bit) : 0u;
-        } else {
-          // all ones where the bit is set: acc, else +0.0f
-#if defined(__HIP_DEVICE_COMPILE__)
-          const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)mine, bit, 1);
-#else
-          const uint32_t keep = ((mine >> bit) & 1u) ? ~0u : 0u;
-#endif
-          v = __uint_as_float(__float_as_uint(acc[i][j][r]) & keep);
-          vals[i][r] = v;
-        }
-        if (ok) Cl[(int64_t)dr * ldc + 32 * j] = v;
-      }
-      if constexpr (EPI == kEpiBiasReluBits) {
-        w <<= 4 * h;
-        w |= partner_u32(w);
-        const int64_t rows = M - (r0 + 32 * i);  // rows of this word inside C
-        if (rows < 32) w &= (1u << (rows > 0 ? rows : 0)) - 1u;
-        if (h == 0 && rows > 0 && col < N) ep.bits[((r0 + 32 * i) >> 5) * N + col] = w;
-      }
-    }
-    if constexpr (EPI == kEpiMaskBits) {
-      if (!ep.part) continue;  // the mask only
-      // colsum's chunk partial: half h's running sum over its rows (row & 4
-      // == 4h) in row order, i.e. its registers in order, then s0 + s1
-      float s = 0.f;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s += vals[i][r];
-      s += __uint_as_float(partner_u32(__float_as_uint(s)));
-      if (h == 0 && col < N && r0 < M) ep.part[(r0 >> 6) * N + col] = s;
-    }
-  }
-}
-
-template <int TM, int TN, int EPI, int NQ = 4, bool BATCH = false>
-__device__ __forceinline__ void store_tile(const f32x16 (&acc)[TM][TN], float* __restrict__ C, const GemmEpi& ep,
-                                           const float (&bias)[TN], int64_t M, int64_t N, int64_t ldc, int64_t r0,
-                                           int64_t c0, int lr, int h, int q0 = 0) {
-  const bool interior = r0 + 32 * TM <= M && c0 + 32 * TN <= N;
-  const int64_t lane0 = (r0 + 4 * h) * ldc + c0 + lr;  // offset of the lane's first element
-  float* const Cl = C + lane0;
-  constexpr bool kAux = EPI == kEpiMask || EPI == kEpiAdd || EPI == kEpiBiasAdd;
-  // The loaded operands (bias, aux) are waited for once, explicitly, before
-  // the stores.  Left to the compiler, the per-element bounds branches made
-  // it wait for vmcnt(0) before every store that uses one (stores count in
-  // vmcnt), one memory round trip per element: measured +10 us on a
-  // 16384 x 1536 x 384 product with the bias epilogue.
-  if constexpr (epi_has_bias(EPI)) wait_vm_lgkm0<0>();
-  const float* const Xl = kAux ? ep.aux + lane0 : nullptr;
-  // The aux values are loaded before any store they feed: C and aux may
-  // alias (an in-place residual), so a load placed after a store would wait
-  // for it, one memory round trip per element.  (Each element is read and
-  // then written by the same lane, so an aliased aux still reads the old
-  // values.)  BATCH (the DMA kernels, whose staging registers are free by
-  // the epilogue): when the wave tile's aux values fit in 96 registers (the
-  // accumulators' count for a 64 x 96 wave tile), all rows of blocks are
-  // loaded in one batch and waited for once, one memory round trip per wave
-  // instead of one per row of blocks.  Otherwise a row of blocks at a time
-  // (in the register path the batch cost occupancy).
-  constexpr int kRowsPerBatch = BATCH && kAux && TM * TN * 4 * NQ <= 96 ? TM : 1;
-  auto load_aux = [&](int i, float (&xv)[TN][4 * NQ]) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int64_t col = c0 + 32 * j + lr;
-#pragma unroll
-      for (int r = 0; r < 4 * NQ; ++r) {
-        const int dr = 32 * i + 8 * (q0 + r / 4) + (r % 4);
-        const int64_t off = (int64_t)dr * ldc + 32 * j;
-        xv[j][r] = (interior || (r0 + 4 * h + dr < M && col < N)) ? Xl[off] : 0.0f;
-      }
-    }
-  };
-#pragma unroll
-  for (int i0 = 0; i0 < TM; i0 += kRowsPerBatch) {
-    float xv[kRowsPerBatch][TN][4 * NQ];
-    if constexpr (kAux) {
-#pragma unroll
-      for (int ib = 0; ib < kRowsPerBatch; ++ib) load_aux(i0 + ib, xv[ib]);
-      wait_vm_lgkm0<0>();
-    }
-#pragma unroll
-    for (int ib = 0; ib < kRowsPerBatch; ++ib) {
-      const int i = i0 + ib;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int64_t col = c0 + 32 * j + lr;
-        const float b = bias[j];
-#pragma unroll
-        for (int r = 0; r < 4 * NQ; ++r) {
-          const int dr = 32 * i + 8 * (q0 + r / 4) + (r % 4);  // row - r0 - 4h
-          const int64_t off = (int64_t)dr * ldc + 32 * j;
-          if (interior || (r0 + 4 * h + dr < M && col < N)) {
-            float v = acc[i][j][r];
-            if constexpr (EPI == kEpiBias) v = v + b;
-            if constexpr (EPI == kEpiBiasRelu) v = fmaxf(0.0f, v + b);
-            if constexpr (EPI == kEpiMask) v = xv[ib][j][r] > 0.0f ? v : 0.0f;
-            if constexpr (EPI == kEpiAdd) v = v + xv[ib][j][r];
-            if constexpr (EPI == kEpiBiasAdd) v = (v + b) + xv[ib][j][r];
-            Cl[off] = v;
-          }
-        }
-      }
-    }
-  }
-}
 
 // ------------------------------------------------------- register path
 // Operands that are not 16-byte aligned or whose contiguous extent is not a
@@ -1039,6 +769,22 @@ gemm_f32_thin_kernel(const float* __restrict__ A, const float* __restrict__ B, f
   }
 }
 
+// The sum over the splits' partial products, in order, rounded once: summed in
+// fp64 (the reduction is bound by its loads), because a chain of up to 64 fp32
+// additions of like signs costs more than the split's shorter chains save
+// (64 x 64 x 4096, uniform operands: 7.8e-8 of the result in fp32).
+__device__ __forceinline__ f32x4 splitk_sum(const f32x4* __restrict__ W, int64_t stride4, int splits) {
+  const f32x4 w0 = W[0];
+  double s[4] = {w0[0], w0[1], w0[2], w0[3]};
+#pragma unroll 8
+  for (int p = 1; p < splits; ++p) {
+    const f32x4 w = W[p * stride4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[e] += (double)w[e];
+  }
+  return f32x4{(float)s[0], (float)s[1], (float)s[2], (float)s[3]};
+}
+
 // C[i] = sum_s W[s*stride + i], s in order 0..splits-1 (deterministic), four
 // consecutive outputs per thread with 128-bit loads (stride % 4 == 0 and
 // 16-byte aligned W/C); the split loop is unrolled so its loads overlap.
@@ -1056,10 +802,7 @@ splitk_reduce_colsum_kernel(const f32x4* __restrict__ W, f32x4* __restrict__ C, 
   if ((int)blockIdx.x < nb_reduce) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n4) return;
-    f32x4 s = W[i];
-#pragma unroll 8
-    for (int p = 1; p < splits; ++p) s += W[p * stride4 + i];
-    C[i] = s;
+    C[i] = splitk_sum(W + i, stride4, splits);
     return;
   }
   colsum_stage2_block<kCsaCols>(part, colsum, nparts, cols, (int64_t)(blockIdx.x - nb_reduce) * kCsaCols, acc);
@@ -1073,9 +816,7 @@ splitk_reduce_vec_kernel(const f32x4* __restrict__ W, f32x4* __restrict__ C, int
                          int64_t n_cols4) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n4) return;
-  f32x4 s = W[i];
-#pragma unroll 8
-  for (int p = 1; p < splits; ++p) s += W[p * stride4 + i];
+  f32x4 s = splitk_sum(W + i, stride4, splits);
   if (epi == kEpiBias || epi == kEpiBiasRelu || epi == kEpiBiasAdd) s += bias[i % n_cols4];
   if (epi == kEpiBiasRelu) {
 #pragma unroll
@@ -1096,9 +837,10 @@ splitk_reduce_kernel(const float* __restrict__ W, float* __restrict__ C, int64_t
                      int64_t n_cols) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  float s = W[i];
+  double sum = W[i];
 #pragma unroll 8
-  for (int p = 1; p < splits; ++p) s += W[p * stride + i];
+  for (int p = 1; p < splits; ++p) sum += (double)W[p * stride + i];
+  float s = (float)sum;
   if (epi == kEpiBias || epi == kEpiBiasRelu || epi == kEpiBiasAdd) s += bias[i % n_cols];
   if (epi == kEpiBiasRelu) s = fmaxf(0.0f, s);
   if (epi == kEpiMask) s = aux[i] > 0.0f ? s : 0.0f;
@@ -1187,6 +929,8 @@ struct Plan {
   int cfg;
   int splits;
   int64_t k_per_split;
+  double us = 0;     // the cost model's time (tile configurations)
+  SplitPlan split{};  // cfg >= 0: the split-operand kernels run the product
 };
 
 int64_t split_chunk(int64_t K, int splits, int bk) { return ceil_div(ceil_div(K, (int64_t)splits), (int64_t)bk) * bk; }
@@ -1306,7 +1050,7 @@ Plan plan_gemm(int op, int64_t M, int64_t N, int64_t K, size_t ws_bytes, bool al
       if (real_splits > 1) t += 6e-6 + (double)(real_splits + 1) * M * N * 4.0 / 3e12;
       if (t < best_t) {
         best_t = t;
-        best = Plan{c, (int)real_splits, kps};
+        best = Plan{c, (int)real_splits, kps, t * 1e6};
       }
     }
   }
@@ -1329,6 +1073,66 @@ Plan plan_gemm(int op, int64_t M, int64_t N, int64_t K, size_t ws_bytes, bool al
   }
   return best;
 }
+
+// 128-bit loads need 16-byte aligned operands whose contiguous extents and
+// leading dimensions are multiples of 4, and the 32-bit per-thread offsets
+// need BR*ld*4 < 2^32.
+constexpr int64_t kMaxLd = (int64_t(1) << 32) / (4 * 256) - 1;
+bool gemm_vec_ok(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B, int64_t lda,
+                 int64_t ldb) {
+  if (!aligned16(A) || !aligned16(B)) return false;
+  if (lda % 4 != 0 || ldb % 4 != 0 || lda > kMaxLd || ldb > kMaxLd) return false;
+  switch (op) {
+    case AAR_GEMM_NN: return (K % 4 == 0) && (N % 4 == 0);
+    case AAR_GEMM_NT: return (K % 4 == 0);
+    default: return (M % 4 == 0) && (N % 4 == 0);
+  }
+}
+
+int default_ld(int op, int64_t M, int64_t N, int64_t K, int64_t& lda, int64_t& ldb) {
+  switch (op) {
+    case AAR_GEMM_NN: lda = K; ldb = N; break;
+    case AAR_GEMM_NT: lda = K; ldb = K; break;
+    default: lda = M; ldb = N; break;
+  }
+  return AAR_OK;
+}
+
+// Adds to a tile plan the split-operand plan (six bf16 products per fp32 one,
+// gemm_split_kernel.hpp) where that is the faster one: by its model's time
+// against this one's plus 2.5 us of launch (the fp32 model leaves it out), by
+// 7 % at least.  Operands the DMA path cannot stage run the fp32 tiles about
+// 1.35 times slower than the model says (measured 1.3-1.6), contractions of at
+// most 128, which its model has no fixed time for, about 1.3 times.  Measured on MI355X over
+// 147 shape / layout pairs: 0.60-0.79 of the fp32 time from 2048^3 up and on the
+// GPT step's products, 0.35-0.56 on unaligned ones, 0.72-0.98 between 12 and 40
+// us; within 6 % either way below that, which the fp32 plan keeps.  The thin
+// and short kernels keep their products (0.76-1.0 of the split kernels' time).
+Plan with_split(Plan p, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batch, size_t ws_bytes,
+                bool vec) {
+  if (p.cfg >= kNumCfgs) return p;
+  const SplitPlan sp =
+      plan_split_gemm(M, N, K, lda, ldb, batch, ws_bytes, p.splits * (vec ? kCfgs[p.cfg].kg : 1));
+  if (sp.cfg >= 0 && sp.us < 0.93 * (p.us * (!vec ? 1.35 : K <= 128 ? 1.3 : 1.0) + 2.5)) p.split = sp;
+  return p;
+}
+// with_split for contiguous operands.
+Plan with_split(Plan p, int op, int64_t M, int64_t N, int64_t K, size_t ws_bytes, const float* A, const float* B) {
+  int64_t lda, ldb;
+  default_ld(op, M, N, K, lda, ldb);
+  return with_split(p, M, N, K, lda, ldb, 1, ws_bytes, gemm_vec_ok(op, M, N, K, A, B, lda, ldb));
+}
+// Partial products of the split-operand plan with unlimited scratch, whether
+// or not it is the faster one (that also depends on the operands' alignment).
+int split_partials(int op, int64_t M, int64_t N, int64_t K, const Plan& p) {
+  if (p.cfg >= kNumCfgs) return 1;
+  int64_t lda, ldb;
+  default_ld(op, M, N, K, lda, ldb);
+  const int tile = plan_split_gemm(M, N, K, lda, ldb, 1, (size_t)-1, p.splits * kCfgs[p.cfg].kg).splits;
+  return std::max(tile, plan_split_gemm(M, N, K, lda, ldb, 1, (size_t)-1, p.splits).splits);
+}
+// Partial products the plan needs scratch for (1: none).
+int plan_partials(const Plan& p) { return p.split.cfg >= 0 ? p.split.splits : p.splits; }
 
 // Batched launches: `count` matrices at element strides sA / sB / sC.
 struct Batch {
@@ -1440,30 +1244,6 @@ int launch_op(int cfg, bool vec, const float* A, const float* B, float* C, int64
 }
 static_assert(kNumCfgs == 17, "launch_op lists every configuration");
 
-// 128-bit loads need 16-byte aligned operands whose contiguous extents and
-// leading dimensions are multiples of 4, and the 32-bit per-thread offsets
-// need BR*ld*4 < 2^32.
-constexpr int64_t kMaxLd = (int64_t(1) << 32) / (4 * 256) - 1;
-bool gemm_vec_ok(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B, int64_t lda,
-                 int64_t ldb) {
-  if (!aligned16(A) || !aligned16(B)) return false;
-  if (lda % 4 != 0 || ldb % 4 != 0 || lda > kMaxLd || ldb > kMaxLd) return false;
-  switch (op) {
-    case AAR_GEMM_NN: return (K % 4 == 0) && (N % 4 == 0);
-    case AAR_GEMM_NT: return (K % 4 == 0);
-    default: return (M % 4 == 0) && (N % 4 == 0);
-  }
-}
-
-int default_ld(int op, int64_t M, int64_t N, int64_t K, int64_t& lda, int64_t& ldb) {
-  switch (op) {
-    case AAR_GEMM_NN: lda = K; ldb = N; break;
-    case AAR_GEMM_NT: lda = K; ldb = K; break;
-    default: lda = M; ldb = N; break;
-  }
-  return AAR_OK;
-}
-
 int dispatch_op(int op, int cfg, bool vec, const float* A, const float* B, float* C, int64_t M, int64_t N,
                 int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int splits, int64_t kps, int64_t split_stride,
                 const Batch& bt, hipStream_t st, int epi = kEpiNone, const GemmEpi& ep = GemmEpi{}) {
@@ -1532,31 +1312,44 @@ int run_thin(int op, int64_t M, int64_t N, int64_t K, const float* A, const floa
   }
 }
 
+// The product(s) of a plan: the split-operand kernels or the fp32 tiles.
+int dispatch_plan(int op, const Plan& p, const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K,
+                  int64_t lda, int64_t ldb, int64_t ldc, int64_t split_stride, const Batch& bt, hipStream_t st,
+                  int epi = kEpiNone, const GemmEpi& ep = GemmEpi{}) {
+  if (p.split.cfg >= 0) {
+    const GemmEpiArgs e{epi, ep.bias, ep.aux, ep.bits, ep.part};
+    const auto launch = op == AAR_GEMM_NN ? launch_split_nn : op == AAR_GEMM_NT ? launch_split_nt : launch_split_tn;
+    return launch(p.split, A, B, C, M, N, K, lda, ldb, ldc, split_stride, bt.count, bt.sA, bt.sB, bt.sC, e, st);
+  }
+  const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb) && bt.sA % 4 == 0 && bt.sB % 4 == 0;
+  return dispatch_op(op, p.cfg, vec, A, B, C, M, N, K, lda, ldb, ldc, p.splits, p.k_per_split, split_stride, bt, st,
+                     epi, ep);
+}
+
 // epi / ep: the epilogue (kEpi*), applied in an unsplit launch or after the
 // split-K reduction.  C is contiguous (ldc = N), and so is ep.aux.
 int run_gemm(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B, float* C,
              void* workspace, const Plan& p, hipStream_t st, int epi = kEpiNone, const GemmEpi& ep = GemmEpi{}) {
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
-  const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb);
-  float* out = p.splits > 1 ? static_cast<float*>(workspace) : C;
-  const int64_t split_stride = p.splits > 1 ? M * N : 0;
+  const int splits = plan_partials(p);
+  float* out = splits > 1 ? static_cast<float*>(workspace) : C;
+  const int64_t split_stride = splits > 1 ? M * N : 0;
   // kEpiColsumA works in the main loop of every split; the others apply to
   // the finished sum, in the reduction when K is split
-  const int main_epi = p.splits > 1 && epi != kEpiColsumA ? kEpiNone : epi;
-  int rc = dispatch_op(op, p.cfg, vec, A, B, out, M, N, K, lda, ldb, N, p.splits, p.k_per_split, split_stride,
-                       kSingle, st, main_epi, ep);
-  if (rc != AAR_OK || p.splits <= 1) return rc;
+  const int main_epi = splits > 1 && epi != kEpiColsumA ? kEpiNone : epi;
+  int rc = dispatch_plan(op, p, A, B, out, M, N, K, lda, ldb, N, split_stride, kSingle, st, main_epi, ep);
+  if (rc != AAR_OK || splits <= 1) return rc;
   if (epi == kEpiColsumA) epi = kEpiNone;
   const int64_t n = M * N;
   if (n % 4 == 0 && aligned16(out) && aligned16(C) && (!ep.bias || (N % 4 == 0 && aligned16(ep.bias))) &&
       (!ep.aux || aligned16(ep.aux))) {
     splitk_reduce_vec_kernel<<<dim3((unsigned)ceil_div(n / 4, (int64_t)256)), dim3(256), 0, st>>>(
-        reinterpret_cast<const f32x4*>(out), reinterpret_cast<f32x4*>(C), n / 4, split_stride / 4, p.splits, epi,
+        reinterpret_cast<const f32x4*>(out), reinterpret_cast<f32x4*>(C), n / 4, split_stride / 4, splits, epi,
         reinterpret_cast<const f32x4*>(ep.bias), reinterpret_cast<const f32x4*>(ep.aux), N / 4);
   } else {
     splitk_reduce_kernel<<<dim3((unsigned)ceil_div(n, (int64_t)256)), dim3(256), 0, st>>>(
-        out, C, n, split_stride, p.splits, epi, ep.bias, ep.aux, N);
+        out, C, n, split_stride, splits, epi, ep.bias, ep.aux, N);
   }
   return launch_status();
 }
@@ -1594,8 +1387,9 @@ extern "C" size_t aar_gemm_f32_workspace_bytes(int op, int64_t M, int64_t N, int
   if (op < 0 || op > 2 || M <= 0 || N <= 0 || K <= 0) return 0;
   const Plan p = plan_gemm(op, M, N, K, (size_t)-1, true, 1, true, kEpiNone, shape_vec_ok(op, M, N, K));
   if (p.cfg == kShortCfg) return shortm_workspace_bytes(M, N, K, p.splits);
-  if (p.splits <= 1) return 0;
-  return (size_t)p.splits * (size_t)M * (size_t)N * sizeof(float);
+  // the fp32 plan's or the split-operand plan's, whichever is more
+  const int partials = std::max(p.splits, split_partials(op, M, N, K, p));
+  return partials <= 1 ? 0 : (size_t)partials * (size_t)M * (size_t)N * sizeof(float);
 }
 
 extern "C" int aar_gemm_f32(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B,
@@ -1614,6 +1408,7 @@ extern "C" int aar_gemm_f32(int op, int64_t M, int64_t N, int64_t K, const float
     // (an operand alignment the short kernels do not take either)
     p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1, false);
   }
+  p = with_split(p, op, M, N, K, workspace ? workspace_bytes : 0, A, B);
   return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream));
 }
 
@@ -1626,7 +1421,8 @@ extern "C" int aar_gemm_f32_bias(int op, int64_t M, int64_t N, int64_t K, const 
   if (K == 0) return AAR_EUNSUPPORTED;  // C = bias rows: not a product, left to the caller
   const int chk = check_gemm_args(op, M, N, K, A, B, C, stream);
   if (chk != AAR_OK) return chk;
-  const Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1, false, kEpiBias);
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  const Plan p = with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, false, kEpiBias), op, M, N, K, wsb, A, B);
   return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream), kEpiBias, GemmEpi{bias, nullptr});
 }
 
@@ -1639,7 +1435,8 @@ extern "C" int aar_gemm_f32_bias_relu(int op, int64_t M, int64_t N, int64_t K, c
   if (op != AAR_GEMM_NT || K == 0) return AAR_EUNSUPPORTED;
   const int chk = check_gemm_args(op, M, N, K, A, B, C, stream);
   if (chk != AAR_OK) return chk;
-  const Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1, false, kEpiBiasRelu);
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  const Plan p = with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, false, kEpiBiasRelu), op, M, N, K, wsb, A, B);
   return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream), kEpiBiasRelu, GemmEpi{bias, nullptr});
 }
 
@@ -1657,8 +1454,9 @@ extern "C" int aar_gemm_f32_add(int op, int64_t M, int64_t N, int64_t K, const f
   if (chk != AAR_OK) return chk;
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
-  const Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1,
-                           thin_operands_ok(op, A, B, lda, ldb));
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  const Plan p = with_split(
+      plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, thin_operands_ok(op, A, B, lda, ldb)), op, M, N, K, wsb, A, B);
   if (p.cfg == kThinCfg) {
     const int rc = run_thin(op, M, N, K, A, B, C, as_stream(stream));
     return rc != AAR_OK ? rc : aar_add_f32(C, R, C, M * N, stream);
@@ -1677,7 +1475,8 @@ extern "C" int aar_gemm_f32_bias_add(int op, int64_t M, int64_t N, int64_t K, co
   if (op != AAR_GEMM_NT || K == 0) return AAR_EUNSUPPORTED;
   const int chk = check_gemm_args(op, M, N, K, A, B, C, stream);
   if (chk != AAR_OK) return chk;
-  const Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1, false, kEpiBias);
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  const Plan p = with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, false, kEpiBias), op, M, N, K, wsb, A, B);
   return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream), kEpiBiasAdd, GemmEpi{bias, R});
 }
 
@@ -1695,8 +1494,10 @@ extern "C" int aar_gemm_f32_relu_mask(int op, int64_t M, int64_t N, int64_t K, c
   // which has no epilogue, runs the product and then the mask pass
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
-  const Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1,
-                           thin_operands_ok(op, A, B, lda, ldb), kEpiMask);
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  const Plan p =
+      with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiMask),
+                 op, M, N, K, wsb, A, B);
   if (p.cfg == kThinCfg) {
     const int rc = run_thin(op, M, N, K, A, B, C, as_stream(stream));
     return rc != AAR_OK ? rc : aar_relu_bwd_f32(C, mask, C, M * N, stream);
@@ -1716,8 +1517,9 @@ extern "C" int aar_gemm_f32_bias_relu_bits(int op, int64_t M, int64_t N, int64_t
   if (op != AAR_GEMM_NT || K == 0) return AAR_EUNSUPPORTED;
   const int chk = check_gemm_args(op, M, N, K, A, B, C, stream);
   if (chk != AAR_OK) return chk;
-  const Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1, false, kEpiBiasRelu);
-  if (p.splits > 1) return AAR_EUNSUPPORTED;
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  const Plan p = with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, false, kEpiBiasRelu), op, M, N, K, wsb, A, B);
+  if (plan_partials(p) > 1) return AAR_EUNSUPPORTED;
   GemmEpi ep{bias, nullptr};
   ep.bits = bits;
   return run_gemm(op, M, N, K, A, B, C, nullptr, p, as_stream(stream), kEpiBiasReluBits, ep);
@@ -1749,8 +1551,10 @@ extern "C" int aar_gemm_f32_mask_bits_colsum(int op, int64_t M, int64_t N, int64
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
   const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb);
-  const Plan p = plan_gemm(op, M, N, K, (size_t)-1, true, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiMaskBits, vec);
-  if (p.splits > 1 || p.cfg >= kNumCfgs) return AAR_EUNSUPPORTED;
+  const Plan p = with_split(
+      plan_gemm(op, M, N, K, (size_t)-1, true, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiMaskBits, vec), op, M, N, K,
+      (size_t)-1, A, B);
+  if (plan_partials(p) > 1 || p.cfg >= kNumCfgs) return AAR_EUNSUPPORTED;
   GemmEpi ep{nullptr, nullptr};
   ep.bits = const_cast<uint32_t*>(bits);
   ep.part = colsum ? static_cast<float*>(workspace) : nullptr;  // no colsum: the mask only
@@ -1770,10 +1574,11 @@ Plan colsum_a_plan(int op, int64_t M, int64_t N, int64_t K, const float* A, cons
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
   vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb);
-  return plan_gemm(op, M, N, K, (size_t)-1, true, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiNone, vec);
+  return with_split(plan_gemm(op, M, N, K, (size_t)-1, true, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiNone, vec), op,
+                    M, N, K, (size_t)-1, A, B);
 }
-size_t colsum_a_split_bytes(const Plan& p, int64_t M, int64_t N) {
-  return p.splits > 1 ? ceil_div((int64_t)p.splits * M * N * (int64_t)sizeof(float), (int64_t)256) * 256 : 0;
+size_t colsum_a_split_bytes(int partials, int64_t M, int64_t N) {
+  return partials > 1 ? ceil_div((int64_t)partials * M * N * (int64_t)sizeof(float), (int64_t)256) * 256 : 0;
 }
 }  // namespace
 }  // namespace aar
@@ -1782,7 +1587,8 @@ extern "C" size_t aar_gemm_f32_colsum_a_workspace_bytes(int op, int64_t M, int64
   if (op != AAR_GEMM_TN || M <= 0 || N <= 0 || K <= 0) return 0;
   bool vec;
   const Plan p = colsum_a_plan(op, M, N, K, nullptr, nullptr, vec);  // the shape's plan (aligned operands)
-  return colsum_a_split_bytes(p, M, N) + (size_t)ceil_div(K, (int64_t)64) * (size_t)M * sizeof(float);
+  const int partials = std::max(p.splits, split_partials(op, M, N, K, p));  // (the operands' alignment may pick either)
+  return colsum_a_split_bytes(partials, M, N) + (size_t)ceil_div(K, (int64_t)64) * (size_t)M * sizeof(float);
 }
 
 extern "C" int aar_gemm_f32_colsum_a(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B,
@@ -1796,8 +1602,10 @@ extern "C" int aar_gemm_f32_colsum_a(int op, int64_t M, int64_t N, int64_t K, co
   if (chk != AAR_OK) return chk;
   bool vec;
   const Plan p = colsum_a_plan(op, M, N, K, A, B, vec);
-  if (!vec || p.cfg >= kNumCfgs || p.k_per_split % 64 != 0) return AAR_EUNSUPPORTED;
-  const size_t split_bytes = colsum_a_split_bytes(p, M, N);
+  // (the split-operand kernels take any alignment, and their K chunks are whole)
+  if (p.split.cfg < 0 && (!vec || p.cfg >= kNumCfgs || p.k_per_split % 64 != 0)) return AAR_EUNSUPPORTED;
+  const int partials = plan_partials(p);
+  const size_t split_bytes = colsum_a_split_bytes(partials, M, N);
   if (!workspace || workspace_bytes < split_bytes + (size_t)(K / 64) * (size_t)M * sizeof(float)) {
     return AAR_EWORKSPACE;
   }
@@ -1805,24 +1613,22 @@ extern "C" int aar_gemm_f32_colsum_a(int op, int64_t M, int64_t N, int64_t K, co
   ep.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + split_bytes);
   hipStream_t st = as_stream(stream);
   const int nparts = (int)(K / 64);
-  float* out = p.splits > 1 ? static_cast<float*>(workspace) : C;
-  if (p.splits <= 1 || !aligned16(C) || !aligned16(workspace)) {
+  float* out = partials > 1 ? static_cast<float*>(workspace) : C;
+  if (partials <= 1 || !aligned16(C) || !aligned16(workspace) || M * N % 4 != 0) {
     const int rc = run_gemm(op, M, N, K, A, B, C, workspace, p, st, kEpiColsumA, ep);
     if (rc != AAR_OK) return rc;
     return colsum_finish(ep.part, colsum, nparts, M, st);
   }
-  // split: the products, then one launch for the split-K sum and colsum's
-  // stage 2 (M * N % 4 == 0: TN on the DMA path has M % 4 == N % 4 == 0)
+  // split: the products, then one launch for the split-K sum and colsum's stage 2
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
   const int64_t split_stride = M * N;
-  int rc = dispatch_op(op, p.cfg, vec, A, B, out, M, N, K, lda, ldb, N, p.splits, p.k_per_split, split_stride,
-                       kSingle, st, kEpiColsumA, ep);
+  int rc = dispatch_plan(op, p, A, B, out, M, N, K, lda, ldb, N, split_stride, kSingle, st, kEpiColsumA, ep);
   if (rc != AAR_OK) return rc;
   const int64_t n4 = M * N / 4;
   const int nb = (int)ceil_div(n4, (int64_t)256);
   splitk_reduce_colsum_kernel<<<dim3((unsigned)(nb + ceil_div(M, (int64_t)kCsaCols))), dim3(256), 0, st>>>(
-      reinterpret_cast<const f32x4*>(out), reinterpret_cast<f32x4*>(C), n4, split_stride / 4, p.splits, nb, ep.part,
+      reinterpret_cast<const f32x4*>(out), reinterpret_cast<f32x4*>(C), n4, split_stride / 4, partials, nb, ep.part,
       colsum, nparts, M);
   return launch_status();
 }
@@ -1885,14 +1691,14 @@ extern "C" int aar_gemm_f32_batched(int op, int64_t batch, int64_t M, int64_t N,
   // that case plans the tile kernels
   Plan p = plan_gemm(op, M, N, K, 0, false, batch, false, kEpiNone, vec);
   if (p.cfg >= kNumCfgs) p = plan_gemm(op, M, N, K, 0, false, batch);
+  p = with_split(p, M, N, K, lda, ldb, batch, 0, vec);
   // Batches ride blockIdx.z (at most 65535 per launch): larger counts go in
   // consecutive launches (offsets keep the 16-byte alignment, strides % 4 == 0).
   constexpr int64_t kMaxGridZ = 65535;
   for (int64_t b0 = 0; b0 < batch; b0 += kMaxGridZ) {
     const int64_t nb = std::min(kMaxGridZ, batch - b0);
-    const int rc = dispatch_op(op, p.cfg, vec, A + b0 * strideA, B + b0 * strideB, C + b0 * strideC, M, N, K, lda,
-                               ldb, ldc, 1, p.k_per_split, 0, Batch{nb, strideA, strideB, strideC},
-                               as_stream(stream));
+    const int rc = dispatch_plan(op, p, A + b0 * strideA, B + b0 * strideB, C + b0 * strideC, M, N, K, lda, ldb, ldc, 0,
+                                 Batch{nb, strideA, strideB, strideC}, as_stream(stream));
     if (rc != AAR_OK) return rc;
   }
   return AAR_OK;

@@ -87,7 +87,10 @@ int aar_event_elapsed_ms(float* ms, void* start, void* stop);
  * the shape runs without split-K). */
 size_t aar_gemm_f32_workspace_bytes(int op, int64_t M, int64_t N, int64_t K);
 
-/* fp32 GEMM on v_mfma_f32_32x32x2f32.  Replaces matmul_cuda /
+/* fp32 GEMM on the matrix cores: v_mfma_f32_32x32x2f32, or, where that is
+ * faster, the bf16 instruction on operands split exactly into three bf16 parts
+ * (six products; rounding errors a third to a half of the fp32 instruction's,
+ * any finite or non-finite operand as there).  Replaces matmul_cuda /
  * matmul_a_bt_cuda / matmul_at_b_cuda (cppsrc/ops/matmul.cpp:10-12) and the
  * raw-pointer launchers matmul_v4_launch / matmul_a_bt_v4_launch /
  * matmul_at_b_v4_launch (cppsrc/ops/matmul.cu:648-650).
@@ -210,10 +213,11 @@ int aar_gemm_f32_batched(int op, int64_t batch, int64_t M, int64_t N, int64_t K,
  * 16-byte aligned) and NN with K <= 128 (unsplit); aar_gemm_f32 plans them
  * for plain products whose rows the tiled kernels cannot stage (not 16-byte
  * aligned: a vocabulary of 65).
- * aar_gemm_f32_plan reports the configuration and split count aar_gemm_f32
- * would use with `workspace_bytes` of scratch (id n for thin outputs such as
+ * aar_gemm_f32_plan reports the fp32 configuration and split count for the
+ * shape with `workspace_bytes` of scratch (id n for thin outputs such as
  * a vocabulary head; aar_gemm_f32 takes it only when the operands' alignment
- * allows).  aar_gemm_f32_with_config runs a given configuration and split-K
+ * allows); aar_gemm_f32 runs it unless the split-operand kernels are faster,
+ * which this access does not cover.  aar_gemm_f32_with_config runs a given configuration and split-K
  * count (needs splits*M*N*4 bytes of workspace when splits > 1, else
  * AAR_EWORKSPACE); results agree with aar_gemm_f32 up to summation order. */
 int aar_gemm_f32_tile_config(int config, int* tile_m, int* tile_n, int* tile_k);

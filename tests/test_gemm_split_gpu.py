@@ -1,0 +1,128 @@
+"""Split-operand products (fp32 operands in three bf16 parts, six products) on
+the MI355X through aar_gemm_f32, at shapes that the planner gives to each of
+their tile configurations: whole tiles, remainders in every extent, contractions
+shorter than and not a multiple of a K tile, K splits, unaligned operands.
+
+Tolerance: the matrix unit rounds once per 16 products, so an output's error is
+a random walk of K / 16 roundings of at most 2^-24 of a partial sum, plus the
+final rounding and the products left out (2^-25 each): normwise
+2^-24 (2 + sqrt(K / 16)) against fp64.
+
+Magnitudes the split does not cover (bf16 underflow and overflow, infinities,
+NaN) go to the fp32 instruction: the same outputs are non-finite as in fp64
+arithmetic and the others as precise."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from devutil import Abi
+
+pytestmark = pytest.mark.gpu
+NN, NT, TN = 0, 1, 2
+f32, f64 = np.float32, np.float64
+
+
+def _product(op, a, b, offset=0):
+    abi = Abi()
+    try:
+        M = a.shape[1] if op == TN else a.shape[0]
+        K = a.shape[0] if op == TN else a.shape[1]
+        N = b.shape[0] if op == NT else b.shape[1]
+        pa, pb, pc = abi.put(a, offset), abi.put(b, offset), abi.empty(M * N)
+        wsb = abi.L.aar_gemm_f32_workspace_bytes(op, M, N, K)
+        abi.check(abi.L.aar_gemm_f32(op, M, N, K, pa, pb, pc, abi.alloc(wsb) if wsb else None, wsb, None))
+        return abi.get(pc, (M, N))
+    finally:
+        abi.free()
+
+
+def _exact(op, a, b):
+    a, b = a.astype(f64), b.astype(f64)
+    return (a.T if op == TN else a) @ (b.T if op == NT else b)
+
+
+def _operands(op, M, N, K, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.standard_normal((K, M) if op == TN else (M, K)).astype(f32)
+    b = rng.standard_normal((N, K) if op == NT else (K, N)).astype(f32)
+    return a, b
+
+
+def _bound(K):
+    return 2.0 ** -24 * (2 + np.sqrt(K / 16))
+
+
+SHAPES = [
+    (4096, 384, 384),    # 128 x 64 and 64 x 64 tiles
+    (4095, 1537, 130),   # 256 x 128 / 128 x 128, a remainder of one in each extent
+    (3000, 1153, 257),   # a ragged K of one element
+    (2049, 1030, 47),    # a contraction of one whole K tile and a ragged one
+    (2500, 2500, 17),    # a ragged K tile only (32 deep) or one and a remainder (16 deep)
+    (1025, 771, 5001),   # K splits, the last one ragged
+    (384, 384, 16384),   # a weight gradient: 128 x 128 tiles, many splits
+    (70, 70, 9000),      # one tile, many splits
+]
+
+
+@pytest.mark.parametrize("op", [NN, NT, TN])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_split_product_against_fp64(gpu, op, shape):
+    M, N, K = shape
+    a, b = _operands(op, M, N, K, seed=M + N + K + op)
+    for offset in (0, 1):  # 16-byte aligned operands, then off by one float
+        c = _product(op, a, b, offset)
+        r = _exact(op, a, b)
+        assert np.linalg.norm(c - r) <= _bound(K) * np.linalg.norm(r), (op, shape, offset)
+        assert np.array_equal(c, _product(op, a, b, offset))  # deterministic
+
+
+@pytest.mark.parametrize("op", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(2049, 1030, 130), (1025, 771, 5001)])
+def test_split_product_magnitudes(gpu, op, shape):
+    """Rows of A and columns of B from 1e-37 to 1e30, and elements of one row
+    from 1e-40 to 1: every row of the result is as precise as its own scale."""
+    M, N, K = shape
+    a, b = _operands(op, M, N, K, seed=7)
+    A, B = (a.T if op == TN else a), (b.T if op == NT else b)  # [M, K], [K, N] views
+    for r, s in ((0, 1e-37), (1, 1e-30), (2, 1e-20), (3, 1e30), (M - 1, 1e-36)):
+        A[r] *= f32(s)
+    A[5] *= (10.0 ** -np.linspace(0, 40, K)).astype(f32)
+    B[:, 1] *= f32(1e-25)
+    A[6], B[:, 2] = 0.0, 0.0
+    with np.errstate(over="ignore", under="ignore"):
+        c, r = _product(op, a, b), _exact(op, a, b)
+    for i in (0, 1, 2, 3, 5, 6, M - 1):
+        keep = np.arange(N) != 1
+        err, ref = np.linalg.norm(c[i, keep] - r[i, keep]), np.linalg.norm(r[i, keep])
+        # (a scale of 1e-37 leaves subnormal operands and results, of 2^-149 steps)
+        assert err <= 2 * _bound(K) * ref + 2.0 ** -149 * (np.sqrt(N) + K), i
+    assert np.linalg.norm(c[10:, 1] - r[10:, 1]) <= 2 * _bound(K) * np.linalg.norm(r[10:, 1])
+    assert not c[6].any() and not c[:, 2].any()
+
+
+@pytest.mark.parametrize("op", [NN, NT, TN])
+def test_split_product_non_finite(gpu, op):
+    M, N, K = 2049, 1030, 130
+    a, b = _operands(op, M, N, K, seed=9)
+    A, B = (a.T if op == TN else a), (b.T if op == NT else b)
+    A[3, 5], A[700, 0], A[M - 1, K - 1] = np.inf, np.nan, -np.inf
+    B[7, 11], B[100, N - 1] = -np.inf, np.nan
+    A[40, 9] = np.finfo(f32).max  # rounds to infinity in bf16, finite in fp32
+    B[9, :] *= f32(1e-3)
+    A[41], B[:, 20] = f32(3e38), f32(3e38)  # overflows to infinity
+    with np.errstate(all="ignore"):
+        c, r = _product(op, a, b), _exact(op, a, b).astype(f32)
+    # (a sum of 3e38 terms of both signs leaves fp32's range on the way, to
+    # either infinity and from there to NaN)
+    ok = np.ones((M, N), bool)
+    ok[41], ok[:, 20] = False, False
+    assert np.array_equal(np.isnan(c) & ok, np.isnan(r) & ok)
+    assert np.array_equal(np.isinf(c) & ok, np.isinf(r) & ok) and np.array_equal(np.sign(c[np.isinf(r) & ok]),
+                                                                                np.sign(r[np.isinf(r) & ok]))
+    assert c[41, 20] == np.inf
+    good = np.isfinite(r) & ok
+    good[40] = False
+    assert np.linalg.norm((c - r)[good]) <= 2 * _bound(K) * np.linalg.norm(r[good])
+    row = np.isfinite(r[40]) & ok[40]
+    assert np.linalg.norm((c - r)[40, row]) <= 2 * _bound(K) * np.linalg.norm(r[40, row].astype(f64))
