@@ -41,6 +41,7 @@
 #include <initializer_list>
 #include <stdint.h>
 
+#include "bf16x3.hpp"
 #include "common.hpp"
 
 namespace aar {
@@ -115,6 +116,7 @@ template <bool SWZ>
 __device__ __forceinline__ int vt_swz(int c, int r) { return SWZ ? r ^ (((c >> 4) & 3) << 2) : r; }
 template <int DP, bool CAUSAL>
 constexpr bool kVtSwizzle = DP == 128 || !CAUSAL;
+
 // The dQ-from-dS pass stages K transposed the same way; there the swizzled
 // layout is faster also for causal d = 64 (T = 4096: 6.47 -> 6.40 ms per
 // fwd+bwd step; T = 1024: -0.6 %), with bit-identical dQ.
@@ -413,6 +415,381 @@ flash_fwd_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__ Lse, i
         f32x4 v = {o[b][4 * g] * inv_l, o[b][4 * g + 1] * inv_l, o[b][4 * g + 2] * inv_l,
                    o[b][4 * g + 3] * inv_l};
         if (dd < d) store4<VEC>(orow + dd, v, d - dd);
+      }
+    }
+    if (h == 0) Lse[(int64_t)bh * T + qi] = (m + log2f(l)) * kLn2;
+  }
+}
+
+// A [32][DP] tile staged transposed for the split products whose reduced-over
+// dimension is the tile's rows (V^T P^T): a thread takes 8 rows of one
+// column, which is one lane's operand of the matrix op.  Planes are
+// [part][octet][column] in 16-byte units.
+template <int DP>
+struct FaKtSplit {
+  static constexpr int kUnits = DP * 4;  // (column, octet of rows)
+  static constexpr int kPer = kUnits / kFaThreads;
+  static_assert(kUnits % kFaThreads == 0, "whole units per thread");
+  static constexpr int kPlanes = 3 * kUnits;  // 16-byte units of a stage
+  float f[kPer][8];
+  float low = INFINITY, high = 0.f;  // smallest nonzero and largest of the units' largest magnitudes
+
+  // Key e of octet o = 2s + h within the tile: acc_row(8s + e, h).
+  __device__ __forceinline__ static int key(int o, int e) {
+    return 16 * (o >> 1) + 8 * (e >> 2) + 4 * (o & 1) + (e & 3);
+  }
+  // Rows past T are clamped onto row T - 1 (their P is 0; an infinite element
+  // sends the wave to the fp32 path) and columns past d onto column d - 1 (they
+  // feed outputs that are not stored), so no load is predicated.  Offsets
+  // within a tile fit 32 bits (`small`) or take the clamped form.
+  uint32_t off[kPer];
+  int64_t row4;  // bytes per row
+  bool small;
+  __device__ __forceinline__ void init(int64_t st, int d, int tid) {
+    row4 = st * 4;
+    small = st < (int64_t(1) << 24);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int u = tid + i * kFaThreads;
+      off[i] = (uint32_t)(key(u / DP, 0) * st + min(u % DP, d - 1)) * 4u;
+    }
+  }
+  __device__ __forceinline__ void load(const float* __restrict__ K, int64_t st, int row0, int T, int d, int tid) {
+    if (row0 + kTile <= T && small) {
+      const char* base = reinterpret_cast<const char*>(K + (int64_t)row0 * st);
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)  // key(o, e) = key(o, 0) + key(0, e)
+          f[i][e] = *reinterpret_cast<const float*>(base + key(0, e) * row4 + off[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int u = tid + i * kFaThreads;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int row = min(row0 + key(u / DP, e), T - 1);
+          f[i][e] = K[(int64_t)row * st + min(u % DP, d - 1)];
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void store(u32x4* s, int tid) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int u = tid + i * kFaThreads;
+      u32x4 parts[3];
+      float m = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t w[3];
+        m = fmaxf(m, fmaxf(fabsf(f[i][2 * e]), fabsf(f[i][2 * e + 1])));
+        bf16_split_pair(f[i][2 * e], f[i][2 * e + 1], w);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) parts[p][e] = w[p];
+      }
+      low = m != 0.f ? fminf(low, m) : low;
+      high = fmaxf(high, m);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) s[p * kUnits + u] = parts[p];
+    }
+  }
+};
+
+// The same for products over the columns (K Q^T): a thread takes 8 columns of
+// one row; planes are [part][octet of columns][row], the octets one unit
+// further apart so that the eight threads of a row store to distinct banks.
+template <int DP>
+struct FaRowSplit {
+  static constexpr int kOcts = DP / 8;
+  static constexpr int kUnits = kTile * kOcts;
+  static_assert(kUnits == kFaThreads, "one unit per thread");
+  static constexpr int kOs = kTile + 1;
+  static constexpr int kPlane = kOcts * kOs;
+  f32x4 f[2];
+  float low = INFINITY, high = 0.f;
+
+  // Rows past T are clamped onto row T - 1 (the caller masks them), columns
+  // past d onto earlier ones (Q is zero there).
+  uint32_t off[2];
+  bool small;
+  __device__ __forceinline__ static int column(int tid, int g, int d) {
+    return min(8 * (tid % kOcts) + 4 * g, d - 4);  // d is a multiple of 4
+  }
+  __device__ __forceinline__ void init(int64_t st, int d, int tid) {
+    small = st < (int64_t(1) << 24);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) off[g] = (uint32_t)(tid / kOcts * st + column(tid, g, d)) * 4u;
+  }
+  __device__ __forceinline__ void load(const float* __restrict__ K, int64_t st, int row0, int T, int d, int tid) {
+    if (row0 + kTile <= T && small) {
+      const char* base = reinterpret_cast<const char*>(K + (int64_t)row0 * st);
+#pragma unroll
+      for (int g = 0; g < 2; ++g) f[g] = *reinterpret_cast<const f32x4*>(base + off[g]);
+    } else {
+      const float* row = K + (int64_t)min(row0 + tid / kOcts, T - 1) * st;
+#pragma unroll
+      for (int g = 0; g < 2; ++g) f[g] = *reinterpret_cast<const f32x4*>(row + column(tid, g, d));
+    }
+  }
+  __device__ __forceinline__ void store(u32x4* s, int tid) {
+    u32x4 parts[3];
+    float m = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = f[e >> 1][2 * (e & 1)], y = f[e >> 1][2 * (e & 1) + 1];
+      uint32_t w[3];
+      m = fmaxf(m, fmaxf(fabsf(x), fabsf(y)));
+      bf16_split_pair(x, y, w);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) parts[p][e] = w[p];
+    }
+    low = m != 0.f ? fminf(low, m) : low;
+    high = fmaxf(high, m);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) s[p * kPlane + (tid % kOcts) * kOs + tid / kOcts] = parts[p];
+  }
+};
+
+// Whether six products of operands whose magnitudes are m (one operand's largest
+// along the sum; 0: all zero) and [low, high] (the other's) sum as in fp32; see
+// bf16x3.hpp.  n: the number of products in a sum.
+__device__ __forceinline__ bool split_covers(float m, float low, float high, int n) {
+  const float kMin = kSplitLow * kSplitLow;     // 2^-100
+  const float kTiny = 8.0779356694631609e-28f;  // 2^-90
+  const float kMax = 8.5070591730234616e37f;    // 2^126
+  if (m > kMax || high > kMax || m * high * (float)n > kMax) return false;
+  return m == 0.f || (m >= kTiny && low >= kTiny && m * low >= kMin);
+}
+
+// Forward on the bf16 matrix cores, every operand in three bf16 parts
+// (bf16x3.hpp): Q is split once into registers, K and V tiles once per workgroup
+// on their way into LDS (double-buffered planes, one barrier per tile), P in the
+// registers the softmax leaves it in.  Two workgroups per CU cover each other's
+// VALU work (splits and softmax, about 450 instructions a tile beside 48 matrix
+// ops), which bounds it: 1700 matrix cycles a tile and wave of about 3500
+// taken at T = 4096.  Unlike flash_fwd_kernel it does not run K a tile ahead:
+// with that, 11 to 61 registers spilled and it took 1.05-1.5 times as long.
+// Measured, flash_fwd_kernel -> this one: causal B8 H12 T4096 d64 1908 -> 1282
+// us, full B4 H5 T777 d40 77 -> 54, full T2048 d64 24 heads 311 -> 187, 128
+// heads 1235 -> 803; O's error against fp64 5.0e-7 -> 2.1e-7 at T = 4096.
+// Head dims 33 to 64 with 128-bit operands and the unsplit key range.
+template <int DP, bool CAUSAL>
+__global__ void __launch_bounds__(kFaThreads, 2)
+flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__ Lse, int T, int d, int H, int nqb,
+                        int BH, float scale_log2) {
+  constexpr int NS = DP / 16;  // matrix-op steps over the head dim
+  constexpr int NB = DP / 32;  // head-dim output blocks
+  using KT = FaRowSplit<DP>;
+  using VT = FaKtSplit<DP>;
+  __shared__ u32x4 ks[2][3 * KT::kPlane];
+  __shared__ u32x4 vs[2][VT::kPlanes];
+  __shared__ uint32_t range[4];  // low and high of K, then V, as bits
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lr = lane & 31, h = lane >> 5;
+  // Longest work first: the last query blocks have the most key tiles.
+  const int qb = CAUSAL ? nqb - 1 - (int)(blockIdx.x / BH) : (int)(blockIdx.x / BH);
+  const int bh = blockIdx.x % BH;
+  const float* __restrict__ Q = Qv.head(bh, H);
+  const float* __restrict__ K = Kv.head(bh, H);
+  const float* __restrict__ V = Vv.head(bh, H);
+  const int q0 = qb * kBlock + wave * kTile;  // first query of this wave
+  const int qi = q0 + lr;                     // this lane's query
+  if (tid < 4) range[tid] = tid & 1 ? 0u : __float_as_uint(INFINITY);
+
+  u32x4 qp[NS][3];
+  float q_max = 0.f;
+#pragma unroll
+  for (int c = 0; c < NS; ++c) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int dd = 16 * c + 8 * h + 4 * g;
+      const f32x4 x = qi < T ? load4<true>(Q + (int64_t)qi * Qv.st + dd, d - dd) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        uint32_t w[3];
+        q_max = fmaxf(fmaxf(q_max, fabsf(x[2 * e])), fabsf(x[2 * e + 1]));
+        bf16_split_pair(x[2 * e], x[2 * e + 1], w);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) qp[c][p][2 * g + e] = w[p];
+      }
+    }
+  }
+  f32x16 o[NB], o_low[NB];  // the hi hi products, and the five smaller ones
+  float m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int b = 0; b < NB; ++b) o[b] = o_low[b] = zero16();
+
+  const int kv_end = CAUSAL ? min(T, qb * kBlock + kBlock) : T;
+  const int ntiles = (kv_end + kTile - 1) / kTile;
+  // Last key tile that holds a key this wave's queries may see.
+  const int wl = CAUSAL ? min(ntiles - 1, (q0 + kTile - 1) / kTile) : ntiles - 1;
+
+  // S^T tile: lane = query, register r = key acc_row(r, h).
+  auto qk = [&](const u32x4* kt) {
+    f32x16 s = zero16(), low = zero16();
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      u32x4 kf[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) kf[p] = kt[p * KT::kPlane + (2 * c + h) * KT::kOs + lr];
+#pragma unroll
+      for (int pr = 0; pr < kSplitProducts; ++pr) {
+        f32x16& a = pr + 1 == kSplitProducts ? s : low;
+        a = mfma_bf16(kf[kSplitA[pr]], qp[c][kSplitB[pr]], a);
+      }
+    }
+    return s + low;
+  };
+  // Online softmax of a tile: S in s becomes P; the factor on O.
+  auto soft = [&](f32x16& s, int kv0) {
+    float mx = -INFINITY;
+    if ((CAUSAL && kv0 + kTile - 1 > q0) || kv0 + kTile > T) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = kv0 + acc_row(r, h);
+        float v = s[r] * scale_log2;
+        if (key >= T || (CAUSAL && key > qi)) v = -INFINITY;
+        s[r] = v;
+        mx = fmaxf(mx, v);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[r] *= scale_log2;
+        mx = fmaxf(mx, s[r]);
+      }
+    }
+    mx = half_swap_max(mx);
+    const float m_new = fmaxf(m, mx);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = fast_exp2(m - m_use);
+    float ps = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = fast_exp2(s[r] - m_use);
+      s[r] = p;
+      ps += p;
+    }
+    ps = half_swap_sum(ps);
+    l = l * alpha + ps;
+    m = m_new;
+    return alpha;
+  };
+  auto soft_pv = [&](f32x16 s, const u32x4* vt, int kv0) {
+    const float alpha = soft(s, kv0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        o[b][r] *= alpha;
+        o_low[b][r] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      u32x4 pp[3];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t w[3];
+        bf16_split_pair(s[8 * k + 2 * e], s[8 * k + 2 * e + 1], w);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) pp[p][e] = w[p];
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        u32x4 vf[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) vf[p] = vt[p * VT::kUnits + (2 * k + h) * DP + 32 * b + lr];
+#pragma unroll
+        for (int pr = 0; pr < kSplitProducts; ++pr) {
+          f32x16& a = pr + 1 == kSplitProducts ? o[b] : o_low[b];
+          a = mfma_bf16(vf[kSplitA[pr]], pp[kSplitB[pr]], a);
+        }
+      }
+    }
+  };
+
+  KT kc;
+  VT vc;
+  kc.init(Kv.st, d, tid);
+  vc.init(Vv.st, d, tid);
+  kc.load(K, Kv.st, 0, T, d, tid);
+  vc.load(V, Vv.st, 0, T, d, tid);
+  kc.store(ks[0], tid);
+  vc.store(vs[0], tid);
+  __syncthreads();
+  for (int t = 0; t < ntiles; ++t) {
+    const bool has_next = t + 1 < ntiles;
+    if (has_next) {
+      kc.load(K, Kv.st, (t + 1) * kTile, T, d, tid);
+      vc.load(V, Vv.st, (t + 1) * kTile, T, d, tid);
+    }
+    if (t <= wl) soft_pv(qk(ks[t & 1]), vs[t & 1], t * kTile);
+    if (has_next) {
+      kc.store(ks[(t + 1) & 1], tid);
+      vc.store(vs[(t + 1) & 1], tid);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b) o[b] += o_low[b];
+
+  // Magnitudes the split does not cover are decided by a query's largest
+  // element and K's units, and by V's units (against P, whose largest element
+  // is 1); such a wave's queries are redone with the fp32 instruction,
+  // straight from HBM.
+  atomicMin(&range[0], __float_as_uint(kc.low));  // >= 0: ordered as their bits
+  atomicMax(&range[1], __float_as_uint(kc.high));
+  atomicMin(&range[2], __float_as_uint(vc.low));
+  atomicMax(&range[3], __float_as_uint(vc.high));
+  __syncthreads();
+  const bool covered =
+      split_covers(fmaxf(q_max, __shfl_xor(q_max, 32)), __uint_as_float(range[0]), __uint_as_float(range[1]), d) &&
+      split_covers(1.f, __uint_as_float(range[2]), __uint_as_float(range[3]), T);
+  if (__any(!covered) && q0 < T) {
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) o[b] = zero16();
+    for (int t = 0; t <= wl; ++t) {
+      const int kv0 = t * kTile;
+      f32x16 s = zero16();
+      for (int c = 0; c < d; c += 2) {
+        const bool on = c + h < d;
+        const float kf = on && kv0 + lr < T ? K[(int64_t)(kv0 + lr) * Kv.st + c + h] : 0.f;
+        const float qf = on && qi < T ? Q[(int64_t)qi * Qv.st + c + h] : 0.f;
+        s = mfma32(kf, qf, s);
+      }
+      const float alpha = soft(s, kv0);
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const int col = b * 32 + lr;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[b][r] *= alpha;
+#pragma unroll
+        for (int st = 0; st < 16; ++st) {
+          const int row = kv0 + acc_row(st, h);
+          const float v = row < T && col < d ? V[(int64_t)row * Vv.st + col] : 0.f;
+          o[b] = mfma32(v, s[st], o[b]);
+        }
+      }
+    }
+  }
+
+  if (qi < T) {
+    const float inv_l = 1.0f / l;
+    float* orow = Ov.head(bh, H) + (int64_t)qi * Ov.st;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int dd = b * 32 + 8 * g + 4 * h;
+        f32x4 v = {o[b][4 * g] * inv_l, o[b][4 * g + 1] * inv_l, o[b][4 * g + 2] * inv_l,
+                   o[b][4 * g + 3] * inv_l};
+        if (dd < d) store4<true>(orow + dd, v, d - dd);
       }
     }
     if (h == 0) Lse[(int64_t)bh * T + qi] = (m + log2f(l)) * kLn2;
@@ -1613,6 +1990,17 @@ int fa_fwd_query_block(int64_t bh, int64_t T, int64_t d, bool causal, bool vec, 
   return (grid <= 2 * slots || (T <= 1024 && grid <= 4 * slots)) ? 64 : kBlock;
 }
 
+// Whether an unsplit d = 64 forward takes the bf16 matrix cores.  Measured on
+// MI355X, time relative to flash_fwd_kernel over grids of 20 to 4000
+// workgroups: full attention T = 32 1.8-2.2, 64 1.3-1.7, 128 1.0-1.27, 192
+// 0.83-1.10, 256 0.78-1.00, 320 0.71-0.92, 384 0.72-0.86, 777 0.62-0.74, 2048
+// 0.59-0.70; causal (d = 40; d = 64 takes the paired or split kernels below
+// about 2000 workgroups) T = 256 0.89-1.07, 384 0.81-1.06, 512 0.72-0.84, 777
+// 0.64-0.77, 2048 0.58-0.72: short rows do not pay for splitting Q and for the
+// longer first tile.  Head dims up to 32 stay: 0.8-1.2, with half the matrix
+// work per split element.
+bool fa_fwd_bf16x3(int64_t T, bool causal) { return T > (causal ? 384 : 256); }
+
 template <int DP, bool C, bool VEC>
 struct FwdLaunch {
   static int run(const FwdArgs& a) {
@@ -1646,6 +2034,13 @@ struct FwdLaunch {
       flash_fwd_kernel<DP, C, VEC, true><<<dim3((unsigned)((nqb + sp.S) * a.BH)), dim3(kFaThreads), 0, a.st>>>(
           a.q, a.k, a.v, a.o, a.lse, a.T, a.d, a.H, nqb, a.BH, a.scale * kLog2e, sp);
     } else {
+      if constexpr (DP == 64 && VEC) {
+        if (fa_fwd_bf16x3(a.T, C)) {
+          flash_fwd_bf16x3_kernel<DP, C><<<dim3((unsigned)(nqb * a.BH)), dim3(kFaThreads), 0, a.st>>>(
+              a.q, a.k, a.v, a.o, a.lse, a.T, a.d, a.H, nqb, a.BH, a.scale * kLog2e);
+          return launch_status();
+        }
+      }
       flash_fwd_kernel<DP, C, VEC, false><<<dim3((unsigned)(nqb * a.BH)), dim3(kFaThreads), 0, a.st>>>(
           a.q, a.k, a.v, a.o, a.lse, a.T, a.d, a.H, nqb, a.BH, a.scale * kLog2e, sp);
     }
