@@ -43,6 +43,7 @@
 
 #include "bf16x3.hpp"
 #include "common.hpp"
+#include "flash_offsets.hpp"
 
 namespace aar {
 namespace {
@@ -116,7 +117,6 @@ template <bool SWZ>
 __device__ __forceinline__ int vt_swz(int c, int r) { return SWZ ? r ^ (((c >> 4) & 3) << 2) : r; }
 template <int DP, bool CAUSAL>
 constexpr bool kVtSwizzle = DP == 128 || !CAUSAL;
-
 // The dQ-from-dS pass stages K transposed the same way; there the swizzled
 // layout is faster also for causal d = 64 (T = 4096: 6.47 -> 6.40 ms per
 // fwd+bwd step; T = 1024: -0.6 %), with bit-identical dQ.
@@ -441,17 +441,18 @@ struct FaKtSplit {
   // Rows past T are clamped onto row T - 1 (their P is 0; an infinite element
   // sends the wave to the fp32 path) and columns past d onto column d - 1 (they
   // feed outputs that are not stored), so no load is predicated.  Offsets
-  // within a tile fit 32 bits (`small`) or take the clamped form.
+  // within a tile fit 32 bits (`small`) or take the clamped form, whose
+  // addresses are 64-bit and signed.
   uint32_t off[kPer];
   int64_t row4;  // bytes per row
   bool small;
   __device__ __forceinline__ void init(int64_t st, int d, int tid) {
     row4 = st * 4;
-    small = st < (int64_t(1) << 24);
+    small = tile_offsets_fit(st);
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int u = tid + i * kFaThreads;
-      off[i] = (uint32_t)(key(u / DP, 0) * st + min(u % DP, d - 1)) * 4u;
+      off[i] = tile_offset(key(u / DP, 0), st, min(u % DP, d - 1));
     }
   }
   __device__ __forceinline__ void load(const float* __restrict__ K, int64_t st, int row0, int T, int d, int tid) {
@@ -518,9 +519,9 @@ struct FaRowSplit {
     return min(8 * (tid % kOcts) + 4 * g, d - 4);  // d is a multiple of 4
   }
   __device__ __forceinline__ void init(int64_t st, int d, int tid) {
-    small = st < (int64_t(1) << 24);
+    small = tile_offsets_fit(st);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) off[g] = (uint32_t)(tid / kOcts * st + column(tid, g, d)) * 4u;
+    for (int g = 0; g < 2; ++g) off[g] = tile_offset(tid / kOcts, st, column(tid, g, d));
   }
   __device__ __forceinline__ void load(const float* __restrict__ K, int64_t st, int row0, int T, int d, int tid) {
     if (row0 + kTile <= T && small) {
