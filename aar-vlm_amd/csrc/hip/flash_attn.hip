@@ -821,7 +821,7 @@ struct FaDmaTile64 {
     const float* base;
     int64_t st;
     uint32_t off[kPerWave];
-    bool small;  // 31 rows of stride st fit the 32-bit lane offsets
+    bool small;  // the tile's rows fit the 32-bit lane offsets
   };
   __device__ __forceinline__ static int lane_row(int wave, int i, int lane) {
     return ((wave * kPerWave + i) * kWave + lane) / kGroups;
@@ -831,14 +831,14 @@ struct FaDmaTile64 {
     return ((u % kGroups) ^ ((u / kGroups) & 15)) * 4;
   }
   __device__ __forceinline__ static Src src(const float* __restrict__ base, int64_t st, int wave, int lane) {
-    Src s{base, st, {}, st < (int64_t(1) << 25)};
+    Src s{base, st, {}, tile_offsets_fit(st)};
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i)
-      s.off[i] = (uint32_t)((lane_row(wave, i, lane) * st + lane_col(wave, i, lane)) * 4);
+    for (int i = 0; i < kPerWave; ++i) s.off[i] = tile_offset(lane_row(wave, i, lane), st, lane_col(wave, i, lane));
     return s;
   }
   // Stages rows row0 .. row0 + 31 of `s`.  A tile inside [0, T) takes the
-  // scalar-base form; one that crosses T clamps its rows onto T - 1.
+  // scalar-base form; one that crosses T clamps its rows onto T - 1, by
+  // signed 64-bit addresses.
   __device__ __forceinline__ static void issue(const Src& s, int row0, int T, float* stage, int wave, int lane) {
     if (row0 + kTile <= T && s.small) {
       const float* tile = s.base + (int64_t)row0 * s.st;

@@ -51,6 +51,7 @@ def test_tile_offsets(tmp_path):
 def test_staged_tiles_ask_for_the_rule():
     text = (HIP_DIR / "flash_attn.hip").read_text()
     assert text.count("small = tile_offsets_fit(st)") == text.count("small = ") == 2
+    assert "Src s{base, st, {}, tile_offsets_fit(st)};" in text  # the DMA-staged tiles
 
 
 def _forward(abi, q, k, v, causal, backwards):
@@ -76,6 +77,43 @@ def test_forward_of_backward_rows(gpu, T, d, causal):
     abi = Abi()
     try:
         for got, want in zip(_forward(abi, q, k, v, causal, True), _forward(abi, q, k, v, causal, False)):
+            np.testing.assert_array_equal(got, want)
+    finally:
+        abi.free()
+
+
+def _step(abi, ops, causal, query_block, key_block, fast, backwards):
+    """O, lse, dQ, dK, dV on the paired 64-row plans (tiles staged by DMA) or
+    the 128-row ones."""
+    bh, T, d = ops[0].shape
+    flip = (lambda x: x[:, ::-1]) if backwards else (lambda x: x)
+    last = 4 * (T - 1) * d if backwards else 0
+    L, s = abi.L, 1.0 / float(np.sqrt(d))
+    pq, pk, pv, pdo = (abi.put(flip(x)) + last for x in ops)
+    po, pl = abi.empty(bh * T * d) + last, abi.empty(bh * T)
+    st = (ctypes.c_int64 * 24)(*([bh * T * d, T * d, -d if backwards else d] * 8))
+    abi.check(L.aar_flash_fwd_strided_plan_f32(pq, pk, pv, po, pl, 1, bh, T, d, st, int(causal), s, query_block, None,
+                                               0, None))
+    wsb = (L.aar_flash_bwd_fast_workspace_bytes(bh, T, d, int(causal)) if fast
+           else L.aar_flash_bwd_workspace_bytes(bh, T, d))
+    grads = [abi.empty(bh * T * d) + last for _ in range(3)]
+    abi.check(L.aar_flash_bwd_strided_plan_f32(pq, pk, pv, po, pl, pdo, *grads, 1, bh, T, d, st, int(causal), s,
+                                               key_block, abi.alloc(wsb), wsb, None))
+    return [flip(abi.get(p - last, (bh, T, d))) for p in (po, *grads)] + [abi.get(pl, (bh, T))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("fast", [False, True])
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("T", [96, 300, 1056])
+def test_step_of_backward_rows(gpu, T, block, fast, causal):
+    rng = np.random.default_rng(T)
+    ops = [rng.standard_normal((3, T, 64)).astype(np.float32) for _ in range(4)]
+    abi = Abi()
+    try:
+        for got, want in zip(_step(abi, ops, causal, block, block, fast, True),
+                             _step(abi, ops, causal, block, block, fast, False)):
             np.testing.assert_array_equal(got, want)
     finally:
         abi.free()
