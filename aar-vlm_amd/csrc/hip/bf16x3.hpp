@@ -20,10 +20,18 @@
 // uniform ones.)  The bf16 unit reaches 1976 TFLOP/s where the fp32 one
 // reaches 139: 329 TFLOP/s of fp32 products.
 //
+// The matrix op takes subnormal bf16 operands and sums subnormal results as
+// they are (measured), so the split is exact wherever an element's last bit
+// is at least 2^-133, bf16's smallest step: for all elements from 2^-110 up.
 // What the split does not cover is handed to the fp32 instruction by the
-// callers: magnitudes whose low parts fall under bf16's smallest normal
-// (flushed), infinities, and magnitudes that round to infinity.  NaN operands
-// give NaN in the same outputs either way.
+// callers: sums that the part a smaller element leaves over reaches
+// (split_loss_floor), infinities, and magnitudes that round to infinity or whose
+// products' sums might (split_overflows).  NaN operands give NaN in the same
+// outputs either way.
+//
+// Operands in several bf16 parts are a published method (G. Henry, P. Tang, A.
+// Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For
+// Higher-Precision Computations", ARITH 2019).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -50,16 +58,29 @@ __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
-// The three bf16 parts of (a, b) as pairs: a in the low halves.
-__device__ __forceinline__ void bf16_split_pair(float a, float b, uint32_t (&p)[3]) {
+// The three bf16 parts of (a, b) as pairs: a in the low halves.  `rem` collects
+// the bits of what the lowest parts are rounded from: every element is held
+// exactly as long as none of its low 16 bits is set.  (An opaque three-way or,
+// v_bitop3_b32: plain ors are reassociated over the whole tile, which kept 12
+// more registers alive in the 256x128 GEMM tile.)
+__device__ __forceinline__ void bf16_split_pair(float a, float b, uint32_t (&p)[3], uint32_t& rem) {
   p[0] = bf16_pair(a, b);
   a -= __uint_as_float(p[0] << 16);
   b -= __uint_as_float(p[0] & 0xffff0000u);
   p[1] = bf16_pair(a, b);
   a -= __uint_as_float(p[1] << 16);
   b -= __uint_as_float(p[1] & 0xffff0000u);
+#if defined(__HIP_DEVICE_COMPILE__)
+  rem = __builtin_amdgcn_bitop3_b32(rem, __float_as_uint(a), __float_as_uint(b), 0xfe);
+#endif
   p[2] = bf16_pair(a, b);
 }
+__device__ __forceinline__ void bf16_split_pair(float a, float b, uint32_t (&p)[3]) {
+  uint32_t rem = 0;
+  bf16_split_pair(a, b, p, rem);
+}
+
+constexpr uint32_t kSplitRemBits = 0xffffu;
 
 // D = A B + C for 32x32 tiles over 16 k: lane (r = lane % 32, h = lane / 32)
 // holds A[r][8h .. 8h+7] and B[8h .. 8h+7][r]; C/D as the fp32 32x32
@@ -90,12 +111,19 @@ __device__ __forceinline__ void lds_barrier() {
 #endif
 }
 
-// Range of magnitudes the split takes without a closer look: operands whose
-// nonzero maxima lie in [kSplitLow, kSplitHigh] neither lose low parts of any
-// weight (a flushed part is below 2^-126, against products of maxima of
-// 2^-100) nor overflow a sum of fewer than 2^27 products.
-constexpr float kSplitLow = 8.8817841970012523e-16f;   // 2^-50
-constexpr float kSplitHigh = 1.1258999068426240e15f;   // 2^50
-__device__ __forceinline__ bool split_plain(float m) { return m == 0.f || (m >= kSplitLow && m <= kSplitHigh); }
+// Sums of fewer than 2^26 products of magnitudes up to this stay finite.
+constexpr float kSplitPlain = 1.1258999068426240e15f;  // 2^50
+// Whether a sum of n products of magnitudes up to ma and mb might leave fp32's
+// range where the exact one does not (2^126 leaves room for the parts' rounding).
+__device__ __forceinline__ bool split_overflows(float ma, float mb, float n) {
+  const float top = 8.5070591730234616e37f;  // 2^126
+  return !(ma <= top && mb <= top && ma * mb * n <= top);
+}
+// The magnitude from which on such a sum does not feel what elements below 2^-110
+// leave over: at most 2^-134 each, so n 2^-134 (ma + mb) in all,
+// which is less than 2^-24 of it.
+__device__ __forceinline__ float split_loss_floor(float ma, float mb, float n) {
+  return n * 7.7037197775489434e-34f * (ma + mb);  // 2^-110
+}
 
 }  // namespace aar

@@ -557,7 +557,7 @@ struct FaRowSplit {
 // along the sum; 0: all zero) and [low, high] (the other's) sum as in fp32; see
 // bf16x3.hpp.  n: the number of products in a sum.
 __device__ __forceinline__ bool split_covers(float m, float low, float high, int n) {
-  const float kMin = kSplitLow * kSplitLow;     // 2^-100
+  const float kMin = 7.8886090522101181e-31f;   // 2^-100
   const float kTiny = 8.0779356694631609e-28f;  // 2^-90
   const float kMax = 8.5070591730234616e37f;    // 2^126
   if (m > kMax || high > kMax || m * high * (float)n > kMax) return false;

@@ -61,13 +61,14 @@ enum : int {
   kEpiMaskBits = 7,
   kEpiColsumA = 8
 };
-// kEpiColsumA is not an epilogue but work in the main loop (TN only): C is
-// stored plainly, and the waves of the first column of waves also sum the
-// staged A tile's columns: part[k / 64][m] = the sum of A[k][m] over the
-// 64-row chunk of k, in aar_colsum_f32's stage-1 order.  A lane holds the
-// k's with k & 4 == 4h of its column in order, i.e. one of that order's two
-// running sums; the halves add them at the chunk's end.  Chunk q is summed by
-// the workgroups with tn == q % tiles_n, so the work spreads over the grid.
+// kEpiColsumA is not an epilogue (TN only): C is stored plainly, and the kernel
+// also sums A's columns: part[k / 64][m] = the sum of A[k][m] over the 64-row
+// chunk of k, in aar_colsum_f32's stage-1 order.  A lane holds the k's with
+// k & 4 == 4h of its column in order, i.e. one of that order's two running sums;
+// the halves add them at the chunk's end.  Chunk q is summed by the workgroups
+// with tn == q % tiles_n, so the work spreads over the grid.  The fp32 tiles do it
+// in the main loop (the first column of waves, from the staged tile), the
+// split-operand ones ahead of it.
 struct GemmEpi {
   const float* bias;
   const float* aux;

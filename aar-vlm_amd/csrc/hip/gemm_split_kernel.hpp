@@ -26,7 +26,7 @@
 //    It costs registers only (and took 2 % off the times over 147 shapes: the
 //    chains of dependent matrix ops are shorter).
 //  * A K tile's matrix ops are cut into slots of WM/32 instructions; the
-//    conversions of the next tile (11 VALU ops per pair of elements), its LDS
+//    conversions of the next tile (13 VALU ops per pair of elements), its LDS
 //    stores, the loads of the one after and the next fragments are spread over
 //    the slots, with scheduling fences between, so that each slot's VALU work
 //    runs under its matrix ops (left to itself the compiler bunched them: 128x192
@@ -40,6 +40,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 
 #include <algorithm>
 #include <type_traits>
@@ -67,7 +68,7 @@ struct SplitTile {
   static constexpr int kPairs = kU * 4;
 
   float f[kU][8];
-  float mx[kU];  // largest magnitude of each unit's row and octets so far
+  float top = 0.f;  // largest magnitude of this thread's elements
   uint32_t off[kU];
   u32x4 parts[3];
 
@@ -94,7 +95,6 @@ struct SplitTile {
       coords(tid + i * NT, row, oct);
       const uint32_t r = (uint32_t)min(row, lim);
       off[i] = (KC ? r * (uint32_t)ld + 8u * oct : 8u * oct * (uint32_t)ld + r) * 4u;
-      mx[i] = 0.f;
     }
   }
 
@@ -134,13 +134,14 @@ struct SplitTile {
     }
   }
 
-  // Splits pair q of this thread's elements; a unit's last pair stores it.
-  __device__ __forceinline__ void pair(u32x4* __restrict__ s, int tid, int q) {
+  // Splits pair q of this thread's elements; a unit's last pair stores it.  rem:
+  // bf16_split_pair's.
+  __device__ __forceinline__ void pair(u32x4* __restrict__ s, int tid, int q, uint32_t& rem) {
     const int i = q >> 2, e = q & 3;
     const float a = f[i][2 * e], b = f[i][2 * e + 1];
-    mx[i] = fmaxf(fmaxf(mx[i], fabsf(a)), fabsf(b));
+    top = fmaxf(fmaxf(top, fabsf(a)), fabsf(b));
     uint32_t w[3];
-    bf16_split_pair(a, b, w);
+    bf16_split_pair(a, b, w, rem);
 #pragma unroll
     for (int p = 0; p < 3; ++p) parts[p][e] = w[p];
     if (e == 3) {
@@ -150,28 +151,12 @@ struct SplitTile {
       for (int p = 0; p < 3; ++p) s[(p * NO + oct) * kOs + row] = parts[p];
     }
   }
-  __device__ __forceinline__ void store(u32x4* __restrict__ s, int tid) {
+  __device__ __forceinline__ void store(u32x4* __restrict__ s, int tid, uint32_t& rem) {
 #pragma unroll
-    for (int q = 0; q < kPairs; ++q) pair(s, tid, q);
+    for (int q = 0; q < kPairs; ++q) pair(s, tid, q, rem);
   }
   __device__ __forceinline__ static u32x4 frag(const u32x4* __restrict__ s, int part, int oct, int row) {
     return s[(part * NO + oct) * kOs + row];
-  }
-
-  __device__ __forceinline__ bool plain() const {
-    bool ok = true;
-#pragma unroll
-    for (int i = 0; i < kU; ++i) ok = ok && split_plain(mx[i]);
-    return ok;
-  }
-  // Largest magnitude of every row into rows[0 .. BR) (zeroed before).
-  __device__ __forceinline__ void row_max(uint32_t* rows, int tid) const {
-#pragma unroll
-    for (int i = 0; i < kU; ++i) {
-      int row, oct;
-      coords(tid + i * NT, row, oct);
-      atomicMax(rows + row, __float_as_uint(mx[i]));  // mx >= 0: ordered as its bits
-    }
   }
 };
 
@@ -209,6 +194,37 @@ __device__ __forceinline__ void fp32_tile(f32x16 (&acc)[TM][TN], const float* __
 #endif
 }
 
+// kEpiColsumA's sums for A column m: lane half h takes the chunk's k with
+// k & 4 == 4h in order, one of aar_colsum_f32's two running sums; chunk q (64
+// rows of A) belongs to the workgroups with tn == q % tiles_n.  Two chunks' loads
+// are in flight together.  Ahead of the K loop, where nothing else holds registers:
+// among the matrix ops the sums cost 12 % (384 x 1536 x 16384 132 us, now 119, the
+// plain product 116; 4096^3 712 -> 658).
+__device__ __forceinline__ void colsum_a(const float* __restrict__ A, int64_t M, int64_t lda, float* __restrict__ part,
+                                         int64_t m, int h, int64_t kbeg, int64_t kend, int tn, int tiles_n) {
+  const int64_t first = kbeg >> 6, last = kend >> 6;
+  const float* col = A + min(m, M - 1) + 4 * h * lda;
+#pragma unroll 1
+  for (int64_t q = first + (tn + tiles_n - first % tiles_n) % tiles_n; q < last; q += 2 * tiles_n) {
+    const int64_t q2 = q + tiles_n < last ? q + tiles_n : q;  // (the same chunk twice at the end)
+    float v[2][32];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const float* p = col + (c ? q2 : q) * 64 * lda;
+#pragma unroll
+      for (int i = 0; i < 32; ++i) v[c][i] = p[(8 * (i / 4) + i % 4) * lda];
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < 32; ++i) s += v[c][i];
+      s += __uint_as_float(partner_u32(__float_as_uint(s)));
+      if (h == 0 && m < M) part[(c ? q2 : q) * M + m] = s;
+    }
+  }
+}
+
 // WPE: waves per SIMD the register allocation must allow.
 template <int BM, int BN, int BK, int WM, int WN, int WPE, bool A_KC, bool B_KC, int EPI>
 __global__ void __launch_bounds__((BM / WM) * (BN / WN) * 64, WPE)
@@ -224,9 +240,10 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
   using TA = SplitTile<BM, BK, NT, A_KC>;
   using TB = SplitTile<BN, BK, NT, B_KC>;
   constexpr int kStage = TA::kUnits + TB::kUnits;
-  static_assert(EPI != kEpiColsumA || (BM <= 32 * NW && 64 % BK == 0), "a wave sums 32 columns of A");
+  static_assert(EPI != kEpiColsumA || BM <= 32 * NW, "a wave sums 32 columns of A");
   __shared__ u32x4 lds[2 * kStage];
-  __shared__ int unplain;
+  __shared__ int unplain, lossy;  // set by any thread: look closer; an element was split inexactly
+  __shared__ uint32_t top[2];     // largest magnitude of A's and of B's elements, as bits
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -246,7 +263,7 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
   A += (int64_t)blockIdx.z * sA;
   B += (int64_t)blockIdx.z * sB;
   C += (int64_t)blockIdx.z * sC;
-  if (tid == 0) unplain = 0;
+  if (tid == 0) unplain = lossy = top[0] = top[1] = 0;
 
   f32x16 acc[TM][TN], low[TM][TN];  // the hi hi products, and the five smaller ones
 #pragma unroll
@@ -258,6 +275,7 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
 
   TA ta;
   TB tb;
+  uint32_t rem = 0;  // what the splits left over, of both operands
   ta.init(lda, m0, M, tid);
   tb.init(ldb, n0, N, tid);
   float bias[TN];
@@ -279,8 +297,13 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
     tb.load(B, ldb, n0, kf);
     kf = min(kf + BK, klast);
   }
-  ta.store(lds, tid);
-  tb.store(lds + TA::kUnits, tid);
+  // While the first tile is on its way: the column sums of A (K and the splits
+  // are multiples of 64, so every chunk is whole).
+  if constexpr (EPI == kEpiColsumA) {
+    if (wave < BM / 32) colsum_a(A, M, lda, ep.part, m0 + 32 * wave + lr, h, kbeg, kend, tn, tiles_n);
+  }
+  ta.store(lds, tid, rem);
+  tb.store(lds + TA::kUnits, tid, rem);
   if (nt > 1) {
     ta.load(A, lda, m0, kf);
     tb.load(B, ldb, n0, kf);
@@ -288,26 +311,11 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
   }
   lds_barrier();
 
-  // kEpiColsumA (no ragged tile: K and the splits are multiples of 64): the
-  // running sum of A column m0 + 32 wave + lr over the chunk's k with
-  // k & 4 == 4h, aar_colsum_f32's order; chunk q is summed by the workgroups
-  // with tn == q % tiles_n (cs_res is the current chunk's residue).  The rows
-  // were staged an iteration ago, so these loads hit the caches.
-  float csum = 0.f;
-  int cs_res = 0;
-  uint32_t cs_off = 0;  // this lane's column and first k, in bytes from a K tile's origin
-  if constexpr (EPI == kEpiColsumA) {
-    cs_res = (int)((kbeg >> 6) % tiles_n);
-    cs_off = ((uint32_t)min<int64_t>(32 * wave + lr, M - m0 - 1) + 4u * h * (uint32_t)lda) * 4u;
-  }
-
   auto tile = [&](int t, auto more_tag) {
     constexpr bool kMore = decltype(more_tag)::value;  // another tile follows
     const u32x4* as = lds + (t & 1) * kStage;
     const u32x4* bs = as + TA::kUnits;
     u32x4* next = lds + ((t + 1) & 1) * kStage;
-    const int64_t k0 = kbeg + (int64_t)t * BK;
-    const bool cs_on = EPI == kEpiColsumA && cs_res == tn && wave < BM / 32;
     // slots of TM matrix ops; the next tile's pairs start at slot kFirst, after
     // the fragments the first slots wait for
     constexpr int kSlots = KS * TN * kSplitProducts;
@@ -354,10 +362,10 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
           for (int p = 0; p < kPairs; ++p) {
             if (kFirst + p * (kSlots - kFirst) / kPairs == s) {
               if (p < TA::kPairs) {
-                ta.pair(next, tid, p);
+                ta.pair(next, tid, p, rem);
                 if ((p & 3) == 3) ta.load_unit(A, lda, m0, kf, p >> 2);
               } else {
-                tb.pair(next + TA::kUnits, tid, p - TA::kPairs);
+                tb.pair(next + TA::kUnits, tid, p - TA::kPairs, rem);
                 if ((p & 3) == 3) tb.load_unit(B, ldb, n0, kf, (p - TA::kPairs) >> 2);
               }
             }
@@ -367,29 +375,6 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
       }
     }
     if constexpr (kMore) kf = min(kf + BK, klast);
-    if constexpr (EPI == kEpiColsumA) {
-      if (cs_on) {
-        // (loaded here rather than ahead of the matrix ops, where the values
-        // would hold registers the 256x128 tile spilled 55 of)
-        float cv[BK / 2];
-#pragma unroll
-        for (int i = 0; i < BK / 2; ++i) {
-          const char* row = reinterpret_cast<const char*>(A + (k0 + 8 * (i / 4) + i % 4) * lda + m0);
-          cv[i] = *reinterpret_cast<const float*>(row + cs_off);
-        }
-#pragma unroll
-        for (int i = 0; i < BK / 2; ++i) csum += cv[i];
-      }
-      if (((k0 + BK) & 63) == 0) {  // the chunk's last K tile
-        if (cs_on) {
-          const float tot = csum + __uint_as_float(partner_u32(__float_as_uint(csum)));
-          const int64_t m = m0 + 32 * wave + lr;
-          if (h == 0 && m < M) ep.part[(k0 >> 6) * M + m] = tot;
-          csum = 0.f;
-        }
-        cs_res = cs_res + 1 == tiles_n ? 0 : cs_res + 1;
-      }
-    }
   };
   for (int t = 0; t < nt - 1; ++t) {
     tile(t, std::true_type{});
@@ -402,31 +387,30 @@ gemm_split_kernel(const float* __restrict__ A, const float* __restrict__ B, floa
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
 
-  // Magnitudes outside the split's plain range, seen by any thread: look at
-  // whole rows, whose maxima decide (a few tiny elements beside ordinary ones
-  // lose nothing that counts), and redo the tile in fp32 where they do.
-  if (!(ta.plain() && tb.plain())) unplain = 1;
+  // Operands that the split might not cover, seen by any thread: where the sums
+  // might overflow, or a wave's smallest output feels a remainder left over, the
+  // wave's tile is done again in fp32.
+  const bool loss = (rem & kSplitRemBits) != 0;
+  if (loss || !(ta.top <= kSplitPlain && tb.top <= kSplitPlain)) unplain = 1;
+  if (loss) lossy = 1;
   lds_barrier();
   if (unplain) {
-    uint32_t* rows = reinterpret_cast<uint32_t*>(lds);
-    for (int i = tid; i < BM + BN; i += NT) rows[i] = 0u;
+    atomicMax(&top[0], __float_as_uint(ta.top));  // >= 0: ordered as their bits
+    atomicMax(&top[1], __float_as_uint(tb.top));
     __syncthreads();
-    ta.row_max(rows, tid);
-    tb.row_max(rows + BM, tid);
-    __syncthreads();
-    float low[2] = {kSplitHigh, kSplitHigh}, high[2] = {0.f, 0.f};
-    for (int i = 0; i < BM + BN; ++i) {
-      const float m = __uint_as_float(rows[i]);
-      const int o = i < BM ? 0 : 1;
-      if (m != 0.f) low[o] = fminf(low[o], m);
-      high[o] = fmaxf(high[o], m);
+    const float ma = __uint_as_float(top[0]), mb = __uint_as_float(top[1]), n = (float)(kend - kbeg);
+    bool redo = split_overflows(ma, mb, n);
+    if (!redo && lossy) {
+      float least = INFINITY;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) least = fminf(least, fabsf(acc[i][j][r]));
+      redo = __any(least < split_loss_floor(ma, mb, n));
     }
-    const float kMin = kSplitLow * kSplitLow;       // 2^-100
-    const float kTiny = 8.0779356694631609e-28f;    // 2^-90
-    const float kMax = 8.5070591730234616e37f;      // 2^126
-    const bool ok = low[0] >= kTiny && low[1] >= kTiny && low[0] * low[1] >= kMin && high[0] <= kMax &&
-                    high[1] <= kMax && high[0] * high[1] * (float)(kend - kbeg) <= kMax;
-    if (!ok) fp32_tile<TM, TN, A_KC, B_KC>(acc, A, B, M, N, lda, ldb, m0 + wm0, n0 + wn0, kbeg, kend, lr, h);
+    if (redo) fp32_tile<TM, TN, A_KC, B_KC>(acc, A, B, M, N, lda, ldb, m0 + wm0, n0 + wn0, kbeg, kend, lr, h);
   }
 
   if constexpr (epi_bits(EPI)) {

@@ -89,8 +89,10 @@ size_t aar_gemm_f32_workspace_bytes(int op, int64_t M, int64_t N, int64_t K);
 
 /* fp32 GEMM on the matrix cores: v_mfma_f32_32x32x2f32, or, where that is
  * faster, the bf16 instruction on operands split exactly into three bf16 parts
- * (six products; rounding errors a third to a half of the fp32 instruction's,
- * any finite or non-finite operand as there).  Replaces matmul_cuda /
+ * (six products; rounding errors a third to a half of the fp32 instruction's).
+ * Operands that the parts do not hold (elements below 2^-110 whose loss an
+ * output would feel, infinities, magnitudes whose sums might overflow) take the
+ * fp32 instruction, tile by tile.  Replaces matmul_cuda /
  * matmul_a_bt_cuda / matmul_at_b_cuda (cppsrc/ops/matmul.cpp:10-12) and the
  * raw-pointer launchers matmul_v4_launch / matmul_a_bt_v4_launch /
  * matmul_at_b_v4_launch (cppsrc/ops/matmul.cu:648-650).
@@ -175,8 +177,8 @@ int aar_gemm_f32_mask_bits_colsum(int op, int64_t M, int64_t N, int64_t K, const
  * gradient G: C = A^T B (TN; A = G [K, M], B = the layer input [K, N]) and
  * colsum[m] = sum over k of A[k][m].  C is bit-identical to aar_gemm_f32 given
  * the workspace aar_gemm_f32_workspace_bytes asks for (the same plan), colsum
- * to aar_colsum_f32 over A: the GEMM's main loop sums the A tiles it stages
- * into colsum's per-64-row partials.  The workspace
+ * to aar_colsum_f32 over A: the GEMM's kernel also sums A's columns into
+ * colsum's per-64-row partials.  The workspace
  * (aar_gemm_f32_colsum_a_workspace_bytes) holds the split-K partials and those.
  * Returns AAR_EUNSUPPORTED, launching nothing, for op other than TN, K not a
  * multiple of 64 up to 16384 (colsum's partials are not 64-row chunks there),

@@ -126,3 +126,46 @@ def test_split_product_non_finite(gpu, op):
     assert np.linalg.norm((c - r)[good]) <= 2 * _bound(K) * np.linalg.norm(r[good])
     row = np.isfinite(r[40]) & ok[40]
     assert np.linalg.norm((c - r)[40, row]) <= 2 * _bound(K) * np.linalg.norm(r[40, row].astype(f64))
+
+
+@pytest.mark.parametrize("op", [NN, NT, TN])
+@pytest.mark.parametrize("shape", [(4095, 1537, 130), (2049, 1030, 257), (1025, 771, 5001)])
+@pytest.mark.parametrize("scale", [0, 50, -60])
+def test_split_product_selects_tiny_elements(gpu, op, shape, scale):
+    """Every output is one element of A times a power of two, the elements of a
+    row lying between fp32's smallest subnormal and 1e15: nothing else adds up,
+    so each output is that element's exact product, whatever stands beside it.
+    (At 2^-60 the small ones' products are rounded to subnormals: within one
+    step of 2^-149 per part that is summed.)"""
+    M, N, K = shape
+    rng = np.random.default_rng(M + scale)
+    x = (rng.uniform(1, 2, (M, K)) * 2.0 ** rng.uniform(-150, 50, (M, K)) * rng.choice([-1, 1], (M, K))).astype(f32)
+    x[:, rng.integers(0, K, K // 8)] = 0.0
+    x[::3, 1] = f32(1.0)
+    rows = np.arange(N) % K
+    sel = np.zeros((K, N), f32)
+    sel[rows, np.arange(N)] = f32(2.0 ** scale)
+    a = np.ascontiguousarray(x.T) if op == TN else x
+    b = np.ascontiguousarray(sel.T) if op == NT else sel
+    c, want = _product(op, a, b), x.astype(f64)[:, rows] * 2.0 ** scale
+    if scale >= 0:
+        np.testing.assert_array_equal(c, want)  # (products of a power of two are exact)
+    else:
+        assert (np.abs(c - want) <= 6 * 2.0 ** -149).all()
+        big = np.abs(want) >= 2.0 ** -125  # the parts' products end at 2^-149 or above
+        np.testing.assert_array_equal(c[big], want[big])
+
+
+def test_split_product_tiny_beside_dense(gpu):
+    """Tiny and subnormal elements beside ordinary ones in dense operands, zero
+    rows and columns among them: the outputs feel none of it and stay as
+    precise as without."""
+    M, N, K = 2049, 1030, 257
+    a, b = _operands(NN, M, N, K, seed=11)
+    rng = np.random.default_rng(11)
+    a[rng.random((M, K)) < 0.2] *= f32(1e-36)
+    b[rng.random((K, N)) < 0.2] *= f32(1e-40)
+    a[100:110], b[:, 70:75] = 0.0, 0.0
+    c, r = _product(NN, a, b), _exact(NN, a, b)
+    assert np.linalg.norm(c - r) <= _bound(K) * np.linalg.norm(r)
+    assert not c[100:110].any() and not c[:, 70:75].any()
