@@ -75,11 +75,6 @@ __device__ __forceinline__ void bf16_split_pair(float a, float b, uint32_t (&p)[
 #endif
   p[2] = bf16_pair(a, b);
 }
-__device__ __forceinline__ void bf16_split_pair(float a, float b, uint32_t (&p)[3]) {
-  uint32_t rem = 0;
-  bf16_split_pair(a, b, p, rem);
-}
-
 constexpr uint32_t kSplitRemBits = 0xffffu;
 
 // D = A B + C for 32x32 tiles over 16 k: lane (r = lane % 32, h = lane / 32)

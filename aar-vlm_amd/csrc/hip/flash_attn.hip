@@ -432,14 +432,14 @@ struct FaKtSplit {
   static_assert(kUnits % kFaThreads == 0, "whole units per thread");
   static constexpr int kPlanes = 3 * kUnits;  // 16-byte units of a stage
   float f[kPer][8];
-  float low = INFINITY, high = 0.f;  // smallest nonzero and largest of the units' largest magnitudes
+  float top = 0.f;  // largest magnitude of this thread's elements
 
   // Key e of octet o = 2s + h within the tile: acc_row(8s + e, h).
   __device__ __forceinline__ static int key(int o, int e) {
     return 16 * (o >> 1) + 8 * (e >> 2) + 4 * (o & 1) + (e & 3);
   }
   // Rows past T are clamped onto row T - 1 (their P is 0; an infinite element
-  // sends the wave to the fp32 path) and columns past d onto column d - 1 (they
+  // sends the wave to the fp32 instruction) and columns past d onto column d - 1 (they
   // feed outputs that are not stored), so no load is predicated.  Offsets
   // within a tile fit 32 bits (`small`) or take the clamped form, whose
   // addresses are 64-bit and signed.
@@ -476,22 +476,20 @@ struct FaKtSplit {
       }
     }
   }
-  __device__ __forceinline__ void store(u32x4* s, int tid) {
+  // rem: what the splits left over (bf16_split_pair).
+  __device__ __forceinline__ void store(u32x4* s, int tid, uint32_t& rem) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int u = tid + i * kFaThreads;
       u32x4 parts[3];
-      float m = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         uint32_t w[3];
-        m = fmaxf(m, fmaxf(fabsf(f[i][2 * e]), fabsf(f[i][2 * e + 1])));
-        bf16_split_pair(f[i][2 * e], f[i][2 * e + 1], w);
+        top = fmaxf(fmaxf(top, fabsf(f[i][2 * e])), fabsf(f[i][2 * e + 1]));
+        bf16_split_pair(f[i][2 * e], f[i][2 * e + 1], w, rem);
 #pragma unroll
         for (int p = 0; p < 3; ++p) parts[p][e] = w[p];
       }
-      low = m != 0.f ? fminf(low, m) : low;
-      high = fmaxf(high, m);
 #pragma unroll
       for (int p = 0; p < 3; ++p) s[p * kUnits + u] = parts[p];
     }
@@ -509,7 +507,7 @@ struct FaRowSplit {
   static constexpr int kOs = kTile + 1;
   static constexpr int kPlane = kOcts * kOs;
   f32x4 f[2];
-  float low = INFINITY, high = 0.f;
+  float top = 0.f;
 
   // Rows past T are clamped onto row T - 1 (the caller masks them), columns
   // past d onto earlier ones (Q is zero there).
@@ -534,35 +532,21 @@ struct FaRowSplit {
       for (int g = 0; g < 2; ++g) f[g] = *reinterpret_cast<const f32x4*>(row + column(tid, g, d));
     }
   }
-  __device__ __forceinline__ void store(u32x4* s, int tid) {
+  __device__ __forceinline__ void store(u32x4* s, int tid, uint32_t& rem) {
     u32x4 parts[3];
-    float m = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float x = f[e >> 1][2 * (e & 1)], y = f[e >> 1][2 * (e & 1) + 1];
       uint32_t w[3];
-      m = fmaxf(m, fmaxf(fabsf(x), fabsf(y)));
-      bf16_split_pair(x, y, w);
+      top = fmaxf(fmaxf(top, fabsf(x)), fabsf(y));
+      bf16_split_pair(x, y, w, rem);
 #pragma unroll
       for (int p = 0; p < 3; ++p) parts[p][e] = w[p];
     }
-    low = m != 0.f ? fminf(low, m) : low;
-    high = fmaxf(high, m);
 #pragma unroll
     for (int p = 0; p < 3; ++p) s[p * kPlane + (tid % kOcts) * kOs + tid / kOcts] = parts[p];
   }
 };
-
-// Whether six products of operands whose magnitudes are m (one operand's largest
-// along the sum; 0: all zero) and [low, high] (the other's) sum as in fp32; see
-// bf16x3.hpp.  n: the number of products in a sum.
-__device__ __forceinline__ bool split_covers(float m, float low, float high, int n) {
-  const float kMin = 7.8886090522101181e-31f;   // 2^-100
-  const float kTiny = 8.0779356694631609e-28f;  // 2^-90
-  const float kMax = 8.5070591730234616e37f;    // 2^126
-  if (m > kMax || high > kMax || m * high * (float)n > kMax) return false;
-  return m == 0.f || (m >= kTiny && low >= kTiny && m * low >= kMin);
-}
 
 // Forward on the bf16 matrix cores, every operand in three bf16 parts
 // (bf16x3.hpp): Q is split once into registers, K and V tiles once per workgroup
@@ -574,7 +558,9 @@ __device__ __forceinline__ bool split_covers(float m, float low, float high, int
 // with that, 11 to 61 registers spilled and it took 1.05-1.5 times as long.
 // Measured, flash_fwd_kernel -> this one: causal B8 H12 T4096 d64 1908 -> 1282
 // us, full B4 H5 T777 d40 77 -> 54, full T2048 d64 24 heads 311 -> 187, 128
-// heads 1235 -> 803; O's error against fp64 5.0e-7 -> 2.1e-7 at T = 4096.
+// heads 1235 -> 803; O's error against fp64 5.0e-7 -> 2.1e-7 at T = 4096.  (Since
+// then the check of what the parts hold keeps three registers less alive: 1207 ->
+// 1189, 53.5 -> 50.6, 187 -> 182, 792 -> 774.)
 // Head dims 33 to 64 with 128-bit operands and the unsplit key range.
 template <int DP, bool CAUSAL>
 __global__ void __launch_bounds__(kFaThreads, 2)
@@ -586,7 +572,7 @@ flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__
   using VT = FaKtSplit<DP>;
   __shared__ u32x4 ks[2][3 * KT::kPlane];
   __shared__ u32x4 vs[2][VT::kPlanes];
-  __shared__ uint32_t range[4];  // low and high of K, then V, as bits
+  __shared__ uint32_t range[3];  // largest magnitude of K, of V (as bits), what their splits left over
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lr = lane & 31, h = lane >> 5;
@@ -598,10 +584,11 @@ flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__
   const float* __restrict__ V = Vv.head(bh, H);
   const int q0 = qb * kBlock + wave * kTile;  // first query of this wave
   const int qi = q0 + lr;                     // this lane's query
-  if (tid < 4) range[tid] = tid & 1 ? 0u : __float_as_uint(INFINITY);
+  if (tid < 3) range[tid] = 0u;
 
   u32x4 qp[NS][3];
-  float q_max = 0.f;
+  float q_top = 0.f;
+  uint32_t q_rem = 0, kv_rem = 0, p_rem = 0;  // what the splits left over
 #pragma unroll
   for (int c = 0; c < NS; ++c) {
 #pragma unroll
@@ -611,13 +598,15 @@ flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         uint32_t w[3];
-        q_max = fmaxf(fmaxf(q_max, fabsf(x[2 * e])), fabsf(x[2 * e + 1]));
-        bf16_split_pair(x[2 * e], x[2 * e + 1], w);
+        q_top = fmaxf(fmaxf(q_top, fabsf(x[2 * e])), fabsf(x[2 * e + 1]));
+        bf16_split_pair(x[2 * e], x[2 * e + 1], w, q_rem);
 #pragma unroll
         for (int p = 0; p < 3; ++p) qp[c][p][2 * g + e] = w[p];
       }
     }
   }
+  const bool q_exact = !__any((q_rem & kSplitRemBits) != 0);
+  q_top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(q_top))));
   f32x16 o[NB], o_low[NB];  // the hi hi products, and the five smaller ones
   float m = -INFINITY, l = 0.f;
 #pragma unroll
@@ -695,7 +684,7 @@ flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         uint32_t w[3];
-        bf16_split_pair(s[8 * k + 2 * e], s[8 * k + 2 * e + 1], w);
+        bf16_split_pair(s[8 * k + 2 * e], s[8 * k + 2 * e + 1], w, p_rem);
 #pragma unroll
         for (int p = 0; p < 3; ++p) pp[p][e] = w[p];
       }
@@ -719,8 +708,8 @@ flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__
   vc.init(Vv.st, d, tid);
   kc.load(K, Kv.st, 0, T, d, tid);
   vc.load(V, Vv.st, 0, T, d, tid);
-  kc.store(ks[0], tid);
-  vc.store(vs[0], tid);
+  kc.store(ks[0], tid, kv_rem);
+  vc.store(vs[0], tid, kv_rem);
   __syncthreads();
   for (int t = 0; t < ntiles; ++t) {
     const bool has_next = t + 1 < ntiles;
@@ -730,27 +719,34 @@ flash_fwd_bf16x3_kernel(FaIn Qv, FaIn Kv, FaIn Vv, FaOut Ov, float* __restrict__
     }
     if (t <= wl) soft_pv(qk(ks[t & 1]), vs[t & 1], t * kTile);
     if (has_next) {
-      kc.store(ks[(t + 1) & 1], tid);
-      vc.store(vs[(t + 1) & 1], tid);
+      kc.store(ks[(t + 1) & 1], tid, kv_rem);
+      vc.store(vs[(t + 1) & 1], tid, kv_rem);
     }
     __syncthreads();
   }
 #pragma unroll
   for (int b = 0; b < NB; ++b) o[b] += o_low[b];
 
-  // Magnitudes the split does not cover are decided by a query's largest
-  // element and K's units, and by V's units (against P, whose largest element
-  // is 1); such a wave's queries are redone with the fp32 instruction,
+  // What the split does not cover: sums that might overflow, an element of Q, K or
+  // V that is not held exactly (S decides P by its absolute value, and O may hang
+  // on one row of V), and probabilities below 2^-110 where O is so small that it
+  // feels them.  Such a wave's queries are redone with the fp32 instruction,
   // straight from HBM.
-  atomicMin(&range[0], __float_as_uint(kc.low));  // >= 0: ordered as their bits
-  atomicMax(&range[1], __float_as_uint(kc.high));
-  atomicMin(&range[2], __float_as_uint(vc.low));
-  atomicMax(&range[3], __float_as_uint(vc.high));
+  atomicMax(&range[0], __float_as_uint(kc.top));  // >= 0: ordered as their bits
+  atomicMax(&range[1], __float_as_uint(vc.top));
+  atomicOr(&range[2], kv_rem);
   __syncthreads();
-  const bool covered =
-      split_covers(fmaxf(q_max, __shfl_xor(q_max, 32)), __uint_as_float(range[0]), __uint_as_float(range[1]), d) &&
-      split_covers(1.f, __uint_as_float(range[2]), __uint_as_float(range[3]), T);
-  if (__any(!covered) && q0 < T) {
+  const float v_top = __uint_as_float(range[1]);
+  bool redo = !q_exact || (range[2] & kSplitRemBits) != 0 ||
+              split_overflows(q_top, __uint_as_float(range[0]), (float)d) || split_overflows(1.f, v_top, (float)T);
+  if (__any((p_rem & kSplitRemBits) != 0)) {
+    const float floor = split_loss_floor(v_top, 0.f, (float)T);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) redo = redo || fabsf(o[b][r]) < floor;
+  }
+  if (__any(redo) && q0 < T) {
     m = -INFINITY;
     l = 0.f;
 #pragma unroll
