@@ -848,6 +848,30 @@ splitk_reduce_kernel(const float* __restrict__ W, float* __restrict__ C, int64_t
   C[i] = s;
 }
 
+// splitk_reduce_vec_kernel's bias + relu sums (the same operations), with the
+// relu's mask as bits: a thread takes one column of a 32-row block, which is one
+// word (kEpiBiasReluBits).  Bound by its loads, 256 contiguous bytes a wave.
+__global__ void __launch_bounds__(256)
+splitk_reduce_bits_kernel(const float* __restrict__ W, float* __restrict__ C, int64_t M, int64_t N, int64_t stride,
+                          int splits, const float* __restrict__ bias, uint32_t* __restrict__ bits) {
+  const int64_t tiles_n = (N + 255) / 256;
+  const int64_t block = blockIdx.x / tiles_n, col = (blockIdx.x % tiles_n) * 256 + threadIdx.x;
+  if (col >= N) return;
+  const int rows = (int)min<int64_t>(32, M - 32 * block);
+  uint32_t word = 0u;
+#pragma unroll 4
+  for (int r = 0; r < rows; ++r) {
+    const int64_t i = (32 * block + r) * N + col;
+    double sum = W[i];
+#pragma unroll 4
+    for (int p = 1; p < splits; ++p) sum += (double)W[p * stride + i];
+    const float v = fmaxf(0.0f, (float)sum + bias[col]);
+    C[i] = v;
+    word |= v > 0.0f ? 1u << r : 0u;
+  }
+  bits[block * N + col] = word;
+}
+
 // Tile configurations.  `resident` is the number of workgroups one CU holds
 // (LDS and register budget; it sets the kernel's launch bounds), `stages` the
 // LDS ring depth of the DMA path, `eff` the fraction of the MFMA peak the
@@ -1098,6 +1122,13 @@ int default_ld(int op, int64_t M, int64_t N, int64_t K, int64_t& lda, int64_t& l
   return AAR_OK;
 }
 
+// Whether the fp32 plan of an NN product has the mask-bits epilogue
+// (kEpiMaskBits): the 8-wave 128 x 192 tile does not, but replaces one that does
+// only for products without it.
+bool takes_mask_bits(const Plan& p, bool vec) {
+  return vec && p.splits == 1 && kCfgs[p.cfg].kg == 1 && (kCfgs[p.cfg].wm == 64 || p.cfg == kEightWaveFor8);
+}
+
 // Adds to a tile plan the split-operand plan (six bf16 products per fp32 one,
 // gemm_split_kernel.hpp) where that is the faster one: by its model's time
 // against this one's plus 2.5 us of launch (the fp32 model leaves it out), by
@@ -1108,9 +1139,14 @@ int default_ld(int op, int64_t M, int64_t N, int64_t K, int64_t& lda, int64_t& l
 // GPT step's products, 0.35-0.56 on unaligned ones, 0.72-0.98 between 12 and 40
 // us; within 6 % either way below that, which the fp32 plan keeps.  The thin
 // and short kernels keep their products (0.76-1.0 of the split kernels' time).
-Plan with_split(Plan p, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batch, size_t ws_bytes,
+// An NN product whose fp32 plan has the mask-bits epilogue keeps its K whole, so
+// that aar_gemm_f32_mask_bits_colsum, which has no scratch for partial products,
+// takes it with the plan of aar_gemm_f32: 150 of 59908 shapes scanned, 8 % slower
+// there on average by the model than with K split, 18 % at most.
+Plan with_split(Plan p, int op, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batch, size_t ws_bytes,
                 bool vec) {
   if (p.cfg >= kNumCfgs) return p;
+  if (op == AAR_GEMM_NN && takes_mask_bits(p, vec)) ws_bytes = 0;
   const SplitPlan sp =
       plan_split_gemm(M, N, K, lda, ldb, batch, ws_bytes, p.splits * (vec ? kCfgs[p.cfg].kg : 1));
   if (sp.cfg >= 0 && sp.us < 0.93 * (p.us * (!vec ? 1.35 : K <= 128 ? 1.3 : 1.0) + 2.5)) p.split = sp;
@@ -1120,7 +1156,7 @@ Plan with_split(Plan p, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
 Plan with_split(Plan p, int op, int64_t M, int64_t N, int64_t K, size_t ws_bytes, const float* A, const float* B) {
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
-  return with_split(p, M, N, K, lda, ldb, 1, ws_bytes, gemm_vec_ok(op, M, N, K, A, B, lda, ldb));
+  return with_split(p, op, M, N, K, lda, ldb, 1, ws_bytes, gemm_vec_ok(op, M, N, K, A, B, lda, ldb));
 }
 // Partial products of the split-operand plan with unlimited scratch, whether
 // or not it is the faster one (that also depends on the operands' alignment).
@@ -1342,7 +1378,11 @@ int run_gemm(int op, int64_t M, int64_t N, int64_t K, const float* A, const floa
   if (rc != AAR_OK || splits <= 1) return rc;
   if (epi == kEpiColsumA) epi = kEpiNone;
   const int64_t n = M * N;
-  if (n % 4 == 0 && aligned16(out) && aligned16(C) && (!ep.bias || (N % 4 == 0 && aligned16(ep.bias))) &&
+  if (epi == kEpiBiasReluBits) {
+    const int64_t blocks = ceil_div(M, (int64_t)32) * ceil_div(N, (int64_t)256);
+    splitk_reduce_bits_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(out, C, M, N, split_stride, splits,
+                                                                             ep.bias, ep.bits);
+  } else if (n % 4 == 0 && aligned16(out) && aligned16(C) && (!ep.bias || (N % 4 == 0 && aligned16(ep.bias))) &&
       (!ep.aux || aligned16(ep.aux))) {
     splitk_reduce_vec_kernel<<<dim3((unsigned)ceil_div(n / 4, (int64_t)256)), dim3(256), 0, st>>>(
         reinterpret_cast<const f32x4*>(out), reinterpret_cast<f32x4*>(C), n / 4, split_stride / 4, splits, epi,
@@ -1506,8 +1546,9 @@ extern "C" int aar_gemm_f32_relu_mask(int op, int64_t M, int64_t N, int64_t K, c
 }
 
 // aar_gemm_f32_bias_relu's plan and values, plus the relu's mask as bits
-// (kEpiBiasReluBits).  Plans without that epilogue return AAR_EUNSUPPORTED
-// before anything is launched.
+// (kEpiBiasReluBits; after the split-K reduction where a split-operand plan splits
+// K).  Plans without that epilogue return AAR_EUNSUPPORTED before anything is
+// launched.
 extern "C" int aar_gemm_f32_bias_relu_bits(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B,
                                            const float* bias, float* C, uint32_t* bits, void* workspace,
                                            size_t workspace_bytes, void* stream) {
@@ -1519,10 +1560,10 @@ extern "C" int aar_gemm_f32_bias_relu_bits(int op, int64_t M, int64_t N, int64_t
   if (chk != AAR_OK) return chk;
   const size_t wsb = workspace ? workspace_bytes : 0;
   const Plan p = with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, false, kEpiBiasRelu), op, M, N, K, wsb, A, B);
-  if (plan_partials(p) > 1) return AAR_EUNSUPPORTED;
+  if (p.split.cfg < 0 && p.splits > 1) return AAR_EUNSUPPORTED;
   GemmEpi ep{bias, nullptr};
   ep.bits = bits;
-  return run_gemm(op, M, N, K, A, B, C, nullptr, p, as_stream(stream), kEpiBiasReluBits, ep);
+  return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream), kEpiBiasReluBits, ep);
 }
 
 extern "C" size_t aar_gemm_f32_mask_bits_colsum_workspace_bytes(int64_t M, int64_t N) {
@@ -1691,7 +1732,7 @@ extern "C" int aar_gemm_f32_batched(int op, int64_t batch, int64_t M, int64_t N,
   // that case plans the tile kernels
   Plan p = plan_gemm(op, M, N, K, 0, false, batch, false, kEpiNone, vec);
   if (p.cfg >= kNumCfgs) p = plan_gemm(op, M, N, K, 0, false, batch);
-  p = with_split(p, M, N, K, lda, ldb, batch, 0, vec);
+  p = with_split(p, op, M, N, K, lda, ldb, batch, 0, vec);
   // Batches ride blockIdx.z (at most 65535 per launch): larger counts go in
   // consecutive launches (offsets keep the 16-byte alignment, strides % 4 == 0).
   constexpr int64_t kMaxGridZ = 65535;

@@ -158,11 +158,11 @@ int aar_gemm_f32_relu_mask(int op, int64_t M, int64_t N, int64_t K, const float*
  * aar_colsum_f32; its workspace (aar_gemm_f32_mask_bits_colsum_workspace_bytes)
  * holds colsum's per-64-row partials, which the GEMM epilogue writes.  With
  * colsum NULL it applies the mask only (no workspace).  Both return
- * AAR_EUNSUPPORTED, launching nothing, where the product's plan splits K or
- * has no such epilogue (register staging, K-group tiles, wave tiles of other
- * than 64 rows for the mask) or, for the column sums, where M is not a
- * multiple of 64 up to 16384 (colsum's partials are not 64-row chunks
- * there); the caller then runs the separate passes.  Replace
+ * AAR_EUNSUPPORTED, launching nothing, where the product's plan has no such
+ * epilogue (fp32 plans that split K, register staging, K-group tiles; for the
+ * mask any plan that splits K, and wave tiles of other than 64 rows) or, for the
+ * column sums, where M is not a multiple of 64 up to 16384 (colsum's partials
+ * are not 64-row chunks there); the caller then runs the separate passes.  Replace
  * matmul_a_bt_cuda + add_bias_cuda + relu_cuda and matmul_cuda +
  * relu_backward_cuda + the bias gradient's column sum of the MLP
  * (cppsrc/ops/matmul.cpp:10-11, elementwise.cpp:15-24). */
@@ -182,9 +182,9 @@ int aar_gemm_f32_mask_bits_colsum(int op, int64_t M, int64_t N, int64_t K, const
  * (aar_gemm_f32_colsum_a_workspace_bytes) holds the split-K partials and those.
  * Returns AAR_EUNSUPPORTED, launching nothing, for op other than TN, K not a
  * multiple of 64 up to 16384 (colsum's partials are not 64-row chunks there),
- * or a plan without the path (unaligned operands, the thin or short kernels,
- * K-group tiles, K splits not on 64-row chunks); the caller then runs the two
- * passes.  Replaces matmul_at_b_cuda + bias_grad_cuda of nn.Linear's backward
+ * or a plan without the path (the thin or short kernels; of the fp32 plans those
+ * of unaligned operands, K-group tiles, K splits not on 64-row chunks); the
+ * caller then runs the two passes.  Replaces matmul_at_b_cuda + bias_grad_cuda of nn.Linear's backward
  * (cppsrc/ops/matmul.cpp:12, elementwise.cpp:25). */
 size_t aar_gemm_f32_colsum_a_workspace_bytes(int op, int64_t M, int64_t N, int64_t K);
 int aar_gemm_f32_colsum_a(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B, float* C,

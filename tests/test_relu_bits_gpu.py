@@ -149,6 +149,33 @@ def test_bits_forward_and_masked_backward(gpu, M, H, d, N2):
         abi.free()
 
 
+# (M, N, K) whose fp32 plans take the fused call while the fastest split-operand
+# plan splits K
+SPLIT_K = {NT: [(2048, 2048, 1920), (1280, 3000, 2304), (1025, 3072, 2560), (10000, 300, 2048)],
+           NN: [(2304, 2304, 1920), (2304, 2304, 2560), (1920, 6144, 3072)]}
+
+
+@pytest.mark.parametrize("op,M,N,K", [(op, *s) for op in SPLIT_K for s in SPLIT_K[op]])
+def test_taken_where_k_might_be_split(gpu, op, M, N, K):
+    abi = Abi()
+    L = abi.L
+    _bind(L)
+    try:
+        ones = np.ones(max(M, N) * K, f32)
+        p, q, pc = abi.put(ones[:M * K]), abi.put(ones[:N * K]), abi.empty(M * N)
+        pb, pbits = abi.put(ones[:N]), _sentinel_words(abi, (M + 31) // 32, N)
+        if op == NT:
+            ws = L.aar_gemm_f32_workspace_bytes(NT, M, N, K)
+            w = abi.alloc(ws) if ws else None
+            abi.check(L.aar_gemm_f32_bias_relu_bits(NT, M, N, K, p, q, pb, pc, pbits, w, ws, None))
+        else:
+            abi.check(L.aar_gemm_f32_mask_bits_colsum(NN, M, N, K, p, q, pbits, pc, None, None, 0, None))
+    finally:
+        abi.free()
+    d, N2 = (K, 64) if op == NT else (64, K)
+    test_bits_forward_and_masked_backward(gpu, M, N, d, N2)
+
+
 def test_mask_bits_refusals(gpu):
     """Row counts whose colsum partials are not 64-row chunks, the NT layout
     and a too-small workspace are refused before any launch; zero rows give
