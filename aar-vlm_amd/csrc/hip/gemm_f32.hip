@@ -1592,6 +1592,8 @@ extern "C" int aar_gemm_f32_mask_bits_colsum(int op, int64_t M, int64_t N, int64
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
   const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb);
+  // (aar_gemm_f32 runs such operands on the short-operand kernels, without epilogues)
+  if (!vec && short_plan_ok(op, M, N, K)) return AAR_EUNSUPPORTED;
   const Plan p = with_split(
       plan_gemm(op, M, N, K, (size_t)-1, true, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiMaskBits, vec), op, M, N, K,
       (size_t)-1, A, B);

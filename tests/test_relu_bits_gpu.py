@@ -77,7 +77,7 @@ SHAPES = [
 
 
 @pytest.mark.parametrize("M,H,d,N2", SHAPES)
-def test_bits_forward_and_masked_backward(gpu, M, H, d, N2):
+def test_bits_forward_and_masked_backward(gpu, M, H, d, N2, offset=0):
     rng = np.random.default_rng(M + 7 * H + 13 * d + N2)
     x = rng.standard_normal((M, d)).astype(f32)
     w1 = (rng.standard_normal((H, d)) / np.sqrt(d)).astype(f32)
@@ -89,7 +89,7 @@ def test_bits_forward_and_masked_backward(gpu, M, H, d, N2):
     L = abi.L
     _bind(L)
     try:
-        px, pw1, pb1, pg, pw2 = (abi.put(a) for a in (x, w1, b1, g, w2))
+        px, pw1, pb1, pg, pw2 = (abi.put(a, offset) for a in (x, w1, b1, g, w2))
         wsf = L.aar_gemm_f32_workspace_bytes(NT, M, H, d)
         wf = abi.alloc(wsf) if wsf else None
         # forward: the plain bias + relu product, then the bits entry point
@@ -174,6 +174,19 @@ def test_taken_where_k_might_be_split(gpu, op, M, N, K):
         abi.free()
     d, N2 = (K, 64) if op == NT else (64, K)
     test_bits_forward_and_masked_backward(gpu, M, N, d, N2)
+
+
+# operands that are not 16-byte aligned, or whose rows are not
+UNALIGNED = [(2048, 960, 384, 384, 1), (1024, 771, 385, 257, 0), (4096, 3072, 64, 100, 1), (2304, 2304, 65, 128, 1),
+             (16384, 1023, 131, 96, 1), (4096, 3072, 64, 97, 0), (3072, 8192, 64, 65, 0)]
+
+
+@pytest.mark.parametrize("M,H,d,N2,offset", UNALIGNED)
+def test_bits_of_unaligned_operands(gpu, M, H, d, N2, offset):
+    """Taken or refused, but bit for bit the separate passes' where taken (for a
+    contraction of at most 128 the plain product of such operands runs on the
+    short-operand kernels, which have no epilogue)."""
+    test_bits_forward_and_masked_backward(gpu, M, H, d, N2, offset)
 
 
 def test_mask_bits_refusals(gpu):
