@@ -1137,6 +1137,10 @@ bool takes_mask_bits(const Plan& p, bool vec) {
   return vec && p.splits == 1 && kCfgs[p.cfg].kg == 1 && (kCfgs[p.cfg].wm == 64 || p.cfg == kEightWaveFor8);
 }
 
+// The time below which a split-operand plan replaces tile plan p, whose model is
+// `slow` times too optimistic (with_split).
+double split_limit(const Plan& p, double slow) { return 0.93 * (p.us * slow + 2.5); }
+
 // Adds to a tile plan the split-operand plan (six bf16 products per fp32 one,
 // gemm_split_kernel.hpp) where that is the faster one: by its model's time
 // against this one's plus 2.5 us of launch (the fp32 model leaves it out), by
@@ -1155,9 +1159,8 @@ Plan with_split(Plan p, int op, int64_t M, int64_t N, int64_t K, int64_t lda, in
                 bool vec) {
   if (p.cfg >= kNumCfgs) return p;
   if (op == AAR_GEMM_NN && takes_mask_bits(p, vec)) ws_bytes = 0;
-  const SplitPlan sp =
-      plan_split_gemm(M, N, K, lda, ldb, batch, ws_bytes, p.splits * (vec ? kCfgs[p.cfg].kg : 1));
-  if (sp.cfg >= 0 && sp.us < 0.93 * (p.us * (!vec ? 1.35 : K <= 128 ? 1.3 : 1.0) + 2.5)) p.split = sp;
+  const double limit = split_limit(p, !vec ? 1.35 : K <= 128 ? 1.3 : 1.0);
+  p.split = plan_split_gemm(M, N, K, lda, ldb, batch, ws_bytes, p.splits * (vec ? kCfgs[p.cfg].kg : 1), limit);
   return p;
 }
 // with_split for contiguous operands.
@@ -1166,14 +1169,20 @@ Plan with_split(Plan p, int op, int64_t M, int64_t N, int64_t K, size_t ws_bytes
   default_ld(op, M, N, K, lda, ldb);
   return with_split(p, op, M, N, K, lda, ldb, 1, ws_bytes, gemm_vec_ok(op, M, N, K, A, B, lda, ldb));
 }
-// Partial products of the split-operand plan with unlimited scratch, whether
-// or not it is the faster one (that also depends on the operands' alignment).
+// Partial products of the split-operand plan with unlimited scratch, whether the
+// operands' alignment lets it replace tile plan p (split_limit's largest) and
+// whichever number of chains p has for it (with_split).
 int split_partials(int op, int64_t M, int64_t N, int64_t K, const Plan& p) {
   if (p.cfg >= kNumCfgs) return 1;
   int64_t lda, ldb;
   default_ld(op, M, N, K, lda, ldb);
-  const int tile = plan_split_gemm(M, N, K, lda, ldb, 1, (size_t)-1, p.splits * kCfgs[p.cfg].kg).splits;
-  return std::max(tile, plan_split_gemm(M, N, K, lda, ldb, 1, (size_t)-1, p.splits).splits);
+  const double limit = split_limit(p, 1.35);
+  const int chains = p.splits * kCfgs[p.cfg].kg;
+  int partials = plan_split_gemm(M, N, K, lda, ldb, 1, (size_t)-1, p.splits, limit).splits;
+  // (a plan that also keeps the longer list of chains is the best with it)
+  if (partials * 2 < chains)
+    partials = std::max(partials, plan_split_gemm(M, N, K, lda, ldb, 1, (size_t)-1, chains, limit).splits);
+  return partials;
 }
 // Partial products the plan needs scratch for (1: none).
 int plan_partials(const Plan& p) { return p.split.cfg >= 0 ? p.split.splits : p.splits; }

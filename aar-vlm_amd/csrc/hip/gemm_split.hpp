@@ -55,9 +55,9 @@ struct SplitPlan {
 // separate sums over K that the fp32 plan adds up; this plan keeps at least
 // half of them, so that its rounding error stays the smaller one (over the same
 // K it is 0.33-0.44 of the fp32 instruction's, and errors grow with the square
-// root of a chain's length).
+// root of a chain's length).  limit: plans that take no less are of no use.
 SplitPlan plan_split_gemm(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batch, size_t ws_bytes,
-                          int chains);
+                          int chains, double limit);
 
 // Launch the products of every split into C + split * split_stride.
 // AAR_EUNSUPPORTED, launching nothing, where the configuration lacks the
