@@ -1169,6 +1169,25 @@ Plan with_split(Plan p, int op, int64_t M, int64_t N, int64_t K, size_t ws_bytes
   default_ld(op, M, N, K, lda, ldb);
   return with_split(p, op, M, N, K, lda, ldb, 1, ws_bytes, gemm_vec_ok(op, M, N, K, A, B, lda, ldb));
 }
+// aar_gemm_f32's plan.
+Plan plan_product(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B, size_t ws_bytes,
+                  bool allow_split) {
+  int64_t lda, ldb;
+  default_ld(op, M, N, K, lda, ldb);
+  const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb);
+  return with_split(
+      plan_gemm(op, M, N, K, ws_bytes, allow_split, 1, thin_operands_ok(op, A, B, lda, ldb), kEpiNone, vec), op, M, N,
+      K, lda, ldb, 1, ws_bytes, vec);
+}
+// aar_gemm_f32_batched's: the operands' alignment keeps the DMA-path substitutions
+// off unaligned batches; a short-kernel plan (one unaligned matrix) is not run
+// there, so that case plans the tile kernels.
+Plan plan_batched(int op, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, bool vec) {
+  Plan p = plan_gemm(op, M, N, K, 0, false, batch, false, kEpiNone, vec);
+  if (p.cfg >= kNumCfgs) p = plan_gemm(op, M, N, K, 0, false, batch);
+  return with_split(p, op, M, N, K, lda, ldb, batch, 0, vec);
+}
+
 // Partial products of the split-operand plan with unlimited scratch, whether the
 // operands' alignment lets it replace tile plan p (split_limit's largest) and
 // whichever number of chains p has for it (with_split).
@@ -1453,19 +1472,15 @@ extern "C" int aar_gemm_f32(int op, int64_t M, int64_t N, int64_t K, const float
                             float* C, void* workspace, size_t workspace_bytes, void* stream) {
   const int chk = check_gemm_args(op, M, N, K, A, B, C, stream);
   if (chk != AAR_OK) return chk == 1 ? AAR_OK : chk;
-  int64_t lda, ldb;
-  default_ld(op, M, N, K, lda, ldb);
-  const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb);
-  Plan p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1,
-                     thin_operands_ok(op, A, B, lda, ldb), kEpiNone, vec);
+  const size_t wsb = workspace ? workspace_bytes : 0;
+  Plan p = plan_product(op, M, N, K, A, B, wsb, workspace != nullptr);
   if (p.cfg == kThinCfg) return run_thin(op, M, N, K, A, B, C, as_stream(stream));
   if (p.cfg == kShortCfg) {
     const int rc = run_short(op, M, N, K, A, B, C, p.splits, workspace, workspace_bytes, as_stream(stream));
     if (rc != AAR_EUNSUPPORTED) return rc;
     // (an operand alignment the short kernels do not take either)
-    p = plan_gemm(op, M, N, K, workspace ? workspace_bytes : 0, workspace != nullptr, 1, false);
+    p = with_split(plan_gemm(op, M, N, K, wsb, workspace != nullptr, 1, false), op, M, N, K, wsb, A, B);
   }
-  p = with_split(p, op, M, N, K, workspace ? workspace_bytes : 0, A, B);
   return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream));
 }
 
@@ -1731,6 +1746,45 @@ extern "C" int aar_gemm_f32_with_config(int op, int64_t M, int64_t N, int64_t K,
   return run_gemm(op, M, N, K, A, B, C, workspace, Plan{config, real_splits, kps}, as_stream(stream));
 }
 
+extern "C" int aar_gemm_f32_split_tile_config(int config, int* tile_m, int* tile_n, int* tile_k) {
+  if (config < 0 || config >= kNumSplitCfgs) return AAR_EINVAL;
+  if (tile_m) *tile_m = kSplitCfgs[config].bm;
+  if (tile_n) *tile_n = kSplitCfgs[config].bn;
+  if (tile_k) *tile_k = kSplitCfgs[config].bk;
+  return AAR_OK;
+}
+
+extern "C" int aar_gemm_f32_split_plan(int op, int64_t batch, int64_t M, int64_t N, int64_t K, const float* A,
+                                       const float* B, size_t workspace_bytes, int* config, int* splits) {
+  if (op < 0 || op > 2 || batch < 1 || M <= 0 || N <= 0 || K <= 0) return AAR_EINVAL;
+  int64_t lda, ldb;
+  default_ld(op, M, N, K, lda, ldb);
+  const Plan p = batch == 1 ? plan_product(op, M, N, K, A, B, workspace_bytes, workspace_bytes > 0)
+                            : plan_batched(op, batch, M, N, K, lda, ldb,
+                                           gemm_vec_ok(op, M, N, K, A, B, lda, ldb) && M * K % 4 == 0 && K * N % 4 == 0);
+  if (config) *config = p.split.cfg;
+  if (splits) *splits = p.split.splits;
+  return AAR_OK;
+}
+
+extern "C" int aar_gemm_f32_with_split_config(int op, int64_t M, int64_t N, int64_t K, const float* A, const float* B,
+                                              float* C, void* workspace, size_t workspace_bytes, int config,
+                                              int splits, void* stream) {
+  if (config < 0 || config >= kNumSplitCfgs || splits < 1 || splits > kMaxSplits) return AAR_EINVAL;
+  const int chk = check_gemm_args(op, M, N, K, A, B, C, stream);
+  if (chk != AAR_OK) return chk == 1 ? AAR_OK : chk;
+  int64_t lda, ldb;
+  default_ld(op, M, N, K, lda, ldb);
+  if (lda > kMaxLd || ldb > kMaxLd) return AAR_EUNSUPPORTED;
+  const int64_t kps = splits > 1 ? split_chunk(K, splits, 64) : K;
+  const int real_splits = (int)ceil_div(K, kps);
+  if (real_splits > 1 && (!workspace || workspace_bytes < (size_t)real_splits * M * N * sizeof(float)))
+    return AAR_EWORKSPACE;
+  Plan p{0, real_splits, kps};
+  p.split = SplitPlan{config, real_splits, kps};
+  return run_gemm(op, M, N, K, A, B, C, workspace, p, as_stream(stream));
+}
+
 extern "C" int aar_gemm_f32_batched(int op, int64_t batch, int64_t M, int64_t N, int64_t K, const float* A,
                                     int64_t lda, int64_t strideA, const float* B, int64_t ldb, int64_t strideB,
                                     float* C, int64_t ldc, int64_t strideC, void* stream) {
@@ -1746,12 +1800,7 @@ extern "C" int aar_gemm_f32_batched(int op, int64_t batch, int64_t M, int64_t N,
   if (lda < need_a || ldb < need_b) return AAR_EINVAL;
   if (M > INT32_MAX / 2 || N > INT32_MAX / 2) return AAR_EUNSUPPORTED;
   const bool vec = gemm_vec_ok(op, M, N, K, A, B, lda, ldb) && strideA % 4 == 0 && strideB % 4 == 0;
-  // the operands' alignment keeps the DMA-path substitutions off unaligned
-  // batches; a short-kernel plan (one unaligned matrix) is not run here, so
-  // that case plans the tile kernels
-  Plan p = plan_gemm(op, M, N, K, 0, false, batch, false, kEpiNone, vec);
-  if (p.cfg >= kNumCfgs) p = plan_gemm(op, M, N, K, 0, false, batch);
-  p = with_split(p, op, M, N, K, lda, ldb, batch, 0, vec);
+  const Plan p = plan_batched(op, batch, M, N, K, lda, ldb, vec);
   // Batches ride blockIdx.z (at most 65535 per launch): larger counts go in
   // consecutive launches (offsets keep the 16-byte alignment, strides % 4 == 0).
   constexpr int64_t kMaxGridZ = 65535;

@@ -218,9 +218,9 @@ int aar_gemm_f32_batched(int op, int64_t batch, int64_t M, int64_t N, int64_t K,
  * aar_gemm_f32_plan reports the fp32 configuration and split count for the
  * shape with `workspace_bytes` of scratch (id n for thin outputs such as
  * a vocabulary head; aar_gemm_f32 takes it only when the operands' alignment
- * allows); aar_gemm_f32 runs it unless the split-operand kernels are faster,
- * which this access does not cover.  aar_gemm_f32_with_config runs a given configuration and split-K
- * count (needs splits*M*N*4 bytes of workspace when splits > 1, else
+ * allows); aar_gemm_f32 runs it unless the split-operand kernels are faster
+ * (below).  aar_gemm_f32_with_config runs a given configuration and split-K count
+ * (needs splits*M*N*4 bytes of workspace when splits > 1, else
  * AAR_EWORKSPACE); results agree with aar_gemm_f32 up to summation order. */
 int aar_gemm_f32_tile_config(int config, int* tile_m, int* tile_n, int* tile_k);
 int aar_gemm_f32_plan(int op, int64_t M, int64_t N, int64_t K, size_t workspace_bytes,
@@ -229,6 +229,21 @@ int aar_gemm_f32_with_config(int op, int64_t M, int64_t N, int64_t K,
                              const float* A, const float* B, float* C,
                              void* workspace, size_t workspace_bytes,
                              int config, int splits, void* stream);
+/* The same for the split-operand configurations, numbered 0..n-1 on their own.
+ * aar_gemm_f32_split_plan: the configuration and split count that aar_gemm_f32
+ * (batch 1) or aar_gemm_f32_batched on contiguous matrices (batch > 1, no
+ * workspace) runs the product with; config -1 where it runs aar_gemm_f32_plan's
+ * plan or the short-operand kernels.  Of A and B only the alignment counts; they
+ * are not read.  aar_gemm_f32_with_split_config runs a given one: K in `splits`
+ * chunks of a multiple of 64 (the partial products of more than one need
+ * workspace as above; leading dimensions of 2^22 or more AAR_EUNSUPPORTED). */
+int aar_gemm_f32_split_tile_config(int config, int* tile_m, int* tile_n, int* tile_k);
+int aar_gemm_f32_split_plan(int op, int64_t batch, int64_t M, int64_t N, int64_t K, const float* A, const float* B,
+                            size_t workspace_bytes, int* config, int* splits);
+int aar_gemm_f32_with_split_config(int op, int64_t M, int64_t N, int64_t K,
+                                   const float* A, const float* B, float* C,
+                                   void* workspace, size_t workspace_bytes,
+                                   int config, int splits, void* stream);
 
 /* ------------------------------------------------------- row-wise kernels */
 

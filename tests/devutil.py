@@ -41,6 +41,9 @@ class Abi:
         L.aar_gemm_f32_plan.argtypes = [ctypes.c_int, i64, i64, i64, sz, ip, ip]
         L.aar_gemm_f32_with_config.argtypes = [ctypes.c_int, i64, i64, i64, vp, vp, vp, vp, sz, ctypes.c_int,
                                                ctypes.c_int, vp]
+        L.aar_gemm_f32_split_tile_config.argtypes = [ctypes.c_int, ip, ip, ip]
+        L.aar_gemm_f32_split_plan.argtypes = [ctypes.c_int, i64, i64, i64, i64, vp, vp, sz, ip, ip]
+        L.aar_gemm_f32_with_split_config.argtypes = L.aar_gemm_f32_with_config.argtypes
         L.aar_softmax_fwd_f32.argtypes = [vp, vp, i64, i64, vp]
         L.aar_softmax_bwd_f32.argtypes = [vp, vp, vp, i64, i64, vp]
         L.aar_layernorm_fwd_f32.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, ctypes.c_float, vp]
@@ -98,6 +101,17 @@ class Abi:
         for p in self._bufs:
             self.L.aar_free(p)
         self._bufs.clear()
+
+
+def split_plan(L, op, M, N, K, A=None, B=None, ws=None, batch=1):
+    """(configuration, K splits) of the split-operand plan of a product, or None
+    where it runs on an fp32 plan; A / B addresses count by their alignment (None:
+    aligned), ws None: the workspace the product asks for."""
+    cfg, splits = ctypes.c_int(), ctypes.c_int()
+    ws = L.aar_gemm_f32_workspace_bytes(op, M, N, K) if ws is None else ws
+    rc = L.aar_gemm_f32_split_plan(op, batch, M, N, K, A, B, ws, ctypes.byref(cfg), ctypes.byref(splits))
+    assert rc == 0, rc
+    return None if cfg.value < 0 else (cfg.value, splits.value)
 
 
 def abi_flash(q, k, v, do, causal, query_block=0, key_block=0, fast=True, abi=None):

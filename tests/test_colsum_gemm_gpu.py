@@ -2,9 +2,8 @@
 (aar_gemm_f32_colsum_a, TN): C bit-identical to aar_gemm_f32 with the
 workspace it asks for (the same plan, split or not), colsum bit-identical to
 aar_colsum_f32 over A = G, and within the float64 bound of the exact sums.
-The GPT block's shapes that take the path must take it (the MLP's two weight
-gradients, split 7 ways);
-the others return -3 having written nothing."""
+The GPT block's MLP weight gradients, whose K is split, must take the path; the
+others return -3 having written nothing where they do not."""
 from __future__ import annotations
 
 import ctypes
@@ -32,10 +31,10 @@ def _bind(L):
 
 # (M, N, K, must_take): C[M, N] = A[K, M]^T B[K, N]
 SHAPES = [
-    (384, 1536, 16384, True),   # MLP output layer dW (7 splits)
+    (384, 1536, 16384, True),   # MLP output layer dW (K split)
     (1536, 384, 16384, True),   # MLP input layer dW
-    (384, 384, 16384, False),   # attention out-projection dW (its plan has K groups)
-    (1152, 384, 16384, False),  # qkv dW (its plan has K groups)
+    (384, 384, 16384, False),   # attention out-projection dW
+    (1152, 384, 16384, False),  # qkv dW
     (128, 256, 4096, False),
     (64, 64, 512, False),
     (96, 100, 1024, False),
@@ -43,7 +42,7 @@ SHAPES = [
 
 
 @pytest.mark.parametrize("M,N,K,must", SHAPES)
-def test_colsum_gemm_matches_product_and_colsum(gpu, M, N, K, must):
+def test_colsum_gemm_matches_product_and_colsum(gpu, M, N, K, must, offset=0):
     rng = np.random.default_rng(M + 3 * N + 7 * K)
     a = rng.standard_normal((K, M)).astype(f32)
     b = (rng.standard_normal((K, N)) / np.sqrt(K)).astype(f32)
@@ -51,7 +50,7 @@ def test_colsum_gemm_matches_product_and_colsum(gpu, M, N, K, must):
     L = abi.L
     _bind(L)
     try:
-        pa, pb = abi.put(a), abi.put(b)
+        pa, pb = abi.put(a, offset), abi.put(b, offset)
         wsb = L.aar_gemm_f32_workspace_bytes(TN, M, N, K)
         pc_ref = abi.empty(M * N)
         abi.check(L.aar_gemm_f32(TN, M, N, K, pa, pb, pc_ref, abi.alloc(wsb) if wsb else None, wsb, None))
@@ -75,6 +74,19 @@ def test_colsum_gemm_matches_product_and_colsum(gpu, M, N, K, must):
         assert_close(cs_ref, exact, 1e-6 * np.sqrt(K) * (np.abs(a).sum(0).max() + 1), "colsum vs float64")
     finally:
         abi.free()
+
+
+# operands that are not 16-byte aligned, or whose rows are not; K split and
+# M * N no multiple of 4 in the first three
+UNALIGNED = [(387, 1537, 4096, 0), (1153, 385, 16384, 1), (301, 303, 1024, 0), (384, 1536, 4096, 1), (2047, 2049, 64, 0),
+             (65, 384, 16384, 0)]
+
+
+@pytest.mark.parametrize("M,N,K,offset", UNALIGNED)
+def test_colsum_gemm_of_unaligned_operands(gpu, M, N, K, offset):
+    """Taken or refused (the short-operand kernels' products are), but bit for bit
+    the two passes' where taken."""
+    test_colsum_gemm_matches_product_and_colsum(gpu, M, N, K, M > 260 and K > 64, offset)
 
 
 def test_colsum_gemm_refusals(gpu):

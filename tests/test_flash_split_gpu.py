@@ -142,16 +142,43 @@ def test_tiny_scores(gpu):
     np.testing.assert_allclose(lse[:, :, 0], want, rtol=5e-7)
 
 
+def _plain32(q, k, v, causal):
+    """The formula in float32, for where it is not finite."""
+    with np.errstate(all="ignore"):
+        s = (q @ k.swapaxes(-1, -2)) * f32(1 / math.sqrt(q.shape[-1]))
+        if causal:
+            s = np.where(np.triu(np.ones(s.shape[-2:], bool), 1), f32(-np.inf), s)
+        e = np.exp(s - s.max(-1, keepdims=True))
+        return (e / e.sum(-1, keepdims=True)) @ v
+
+
+@pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("where", ["q", "k", "v"])
 @pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.4e38])
-def test_not_finite(gpu, where, value):
-    # what a query sees of them, as plain float32 gives it; other heads are untouched
-    q, k, v = _inputs(1, 2, 300, 40, 7)
+def test_not_finite(gpu, where, value, causal):
+    """What a query sees of them, as plain float32 gives it.  Other heads, and the
+    queries of earlier tiles under the causal mask, are untouched."""
+    q, k, v = _inputs(1, 2, 400, 40, 7)
+    clean = _exact(q, k, v, causal)[0]
     {"q": q, "k": k, "v": v}[where][0, 0, 40, 3] = value
-    o, _ = _run(gpu, q, k, v, False)
-    _close(o[:, 1:], _exact(q[:, 1:], k[:, 1:], v[:, 1:], False)[0])
+    o, _ = _run(gpu, q, k, v, causal)
+    _close(o[:, 1:], clean[:, 1:])
+    got = o[0, 0]
     if where == "v":
-        hit = o[0, 0, :, 3]
+        # column 3 alone, of the queries that see row 40 (the others of its tile
+        # multiply it by zero)
+        first = 40 if causal else 0
+        hit = got[first:, 3]
         assert np.isnan(hit).all() if np.isnan(value) else ((hit > 1e30) if value > 0 else (hit < -1e30)).all()
-    elif where == "q" and value != f32(3.4e38):
-        assert np.isnan(o[0, 0, 40]).all() and np.isfinite(np.delete(o[0, 0], 40, 0)).all()
+        others = np.delete(got, 3, 1)
+        _close(others[None], np.delete(clean[0, 0], 3, 1)[None])
+        if causal:
+            _close(got[:32], clean[0, 0, :32])
+        return
+    if causal:
+        _close(got[:32 if where == "k" else 40], clean[0, 0, :32 if where == "k" else 40])
+    want = _plain32(q, k, v, causal)[0, 0]
+    bad = ~np.isfinite(want).all(-1)
+    assert bad.any() and np.isnan(got[bad]).all()
+    # (finite scores next to fp32's limit decide the softmax alone: 1e-5 of it)
+    np.testing.assert_allclose(got[~bad], want[~bad], atol=1e-5, rtol=0)

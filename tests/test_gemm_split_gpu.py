@@ -1,7 +1,8 @@
 """Split-operand products (fp32 operands in three bf16 parts, six products) on
-the MI355X through aar_gemm_f32, at shapes that the planner gives to each of
-their tile configurations: whole tiles, remainders in every extent, contractions
-shorter than and not a multiple of a K tile, K splits, unaligned operands.
+the MI355X: through aar_gemm_f32 at shapes that the planner gives to them (which
+the tests ask it), and every tile configuration by itself: whole tiles, remainders
+in every extent, contractions shorter than and not a multiple of a K tile, K
+splits, unaligned operands.
 
 Tolerance: the matrix unit rounds once per 16 products, so an output's error is
 a random walk of K / 16 roundings of at most 2^-24 of a partial sum, plus the
@@ -13,10 +14,12 @@ NaN) go to the fp32 instruction: the same outputs are non-finite as in fp64
 arithmetic and the others as precise."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
-from devutil import Abi
+from devutil import Abi, split_plan
 
 pytestmark = pytest.mark.gpu
 NN, NT, TN = 0, 1, 2
@@ -24,6 +27,7 @@ f32, f64 = np.float32, np.float64
 
 
 def _product(op, a, b, offset=0):
+    """aar_gemm_f32, which must take the split-operand kernels."""
     abi = Abi()
     try:
         M = a.shape[1] if op == TN else a.shape[0]
@@ -31,6 +35,7 @@ def _product(op, a, b, offset=0):
         N = b.shape[0] if op == NT else b.shape[1]
         pa, pb, pc = abi.put(a, offset), abi.put(b, offset), abi.empty(M * N)
         wsb = abi.L.aar_gemm_f32_workspace_bytes(op, M, N, K)
+        assert split_plan(abi.L, op, M, N, K, pa, pb), "this product runs on the fp32 instruction"
         abi.check(abi.L.aar_gemm_f32(op, M, N, K, pa, pb, pc, abi.alloc(wsb) if wsb else None, wsb, None))
         return abi.get(pc, (M, N))
     finally:
@@ -53,18 +58,17 @@ def _bound(K):
     return 2.0 ** -24 * (2 + np.sqrt(K / 16))
 
 
+# every tile configuration is planned by one of them (aligned or off by one float)
 SHAPES = [
-    (4096, 384, 384),    # 128 x 64 and 64 x 64 tiles
-    (4095, 1537, 130),   # 256 x 128 / 128 x 128, a remainder of one in each extent
-    (3000, 1153, 257),   # a ragged K of one element
-    (2049, 1030, 47),    # a contraction of one whole K tile and a ragged one
-    (2500, 2500, 17),    # a ragged K tile only (32 deep) or one and a remainder (16 deep)
+    (2048, 1536, 600),   # 64 x 64 tiles
+    (4095, 1537, 130),   # 256 x 128, a remainder of one in each extent
+    (3000, 1153, 257),   # 128 x 128, a ragged K of one element
+    (8192, 512, 1024),   # 128 x 64
+    (4095, 4097, 65),    # a short contraction: two whole K tiles and a ragged one
     (1025, 771, 5001),   # K splits, the last one ragged
-    (384, 384, 16384),   # a weight gradient: 128 x 128 tiles, many splits
+    (384, 384, 16384),   # a weight gradient: 128 x 192 tiles (unaligned 64 x 128), many splits
     (70, 70, 9000),      # one tile, many splits
 ]
-
-
 @pytest.mark.parametrize("op", [NN, NT, TN])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_split_product_against_fp64(gpu, op, shape):
@@ -169,3 +173,58 @@ def test_split_product_tiny_beside_dense(gpu):
     c, r = _product(NN, a, b), _exact(NN, a, b)
     assert np.linalg.norm(c - r) <= _bound(K) * np.linalg.norm(r)
     assert not c[100:110].any() and not c[:, 70:75].any()
+
+
+def _configs(L):
+    out, tile = [], [ctypes.c_int() for _ in range(3)]
+    while L.aar_gemm_f32_split_tile_config(len(out), *map(ctypes.byref, tile)) == 0:
+        out.append(tuple(t.value for t in tile))
+    return out
+
+
+def test_planned_shapes_cover_the_configurations(gpu):
+    L = Abi().L
+    plans = [split_plan(L, op, *shape, addr, addr) for op in (NN, NT, TN) for shape in SHAPES for addr in (16, 20)]
+    assert {p[0] for p in plans} == set(range(len(_configs(L))))
+    assert any(p[1] > 1 for p in plans) and any(p[1] == 1 for p in plans)
+
+
+@pytest.mark.parametrize("op", [NN, NT, TN])
+@pytest.mark.parametrize("config", range(6))
+def test_every_configuration(gpu, op, config):
+    """Edges of the tiles and of the contraction: K below, at and past one and
+    several K tiles (a ragged tile only, whole tiles only, both), chunks of K whose
+    last one is shorter than a K tile, aligned operands and operands off by one."""
+    abi = Abi()
+    try:
+        tiles = _configs(abi.L)
+        assert len(tiles) == 6
+        bm, bn, bk = tiles[config]
+        cases = [(bm + 1, bn + 1, K, 1) for K in (1, 7, bk - 1, bk, bk + 1, 2 * bk, 2 * bk + 1, 5 * bk - 1)]
+        cases += [(3, 5, 2 * bk + 3, 1), (2 * bm, bn, 3 * bk, 1), (bm - 1, 3 * bn - 31, 4 * bk, 1)]
+        cases += [(bm + 1, bn - 1, 64 * 3 + r, 4) for r in (1, bk - 1, bk, 64)] + [(bm, bn, 128, 2)]
+        for M, N, K, splits in cases:
+            a, b = _operands(op, M, N, K, seed=M + K)
+            for offset in (0, 1):
+                pa, pb, pc = abi.put(a, offset), abi.put(b, offset), abi.put(np.full((M, N), np.nan, f32))
+                ws = 4 * splits * M * N if splits > 1 else 0
+                abi.check(abi.L.aar_gemm_f32_with_split_config(op, M, N, K, pa, pb, pc, abi.alloc(ws) if ws else None,
+                                                               ws, config, splits, None))
+                c, r = abi.get(pc, (M, N)), _exact(op, a, b)
+                assert np.linalg.norm(c - r) <= _bound(K) * np.linalg.norm(r), (M, N, K, splits, offset)
+    finally:
+        abi.free()
+
+
+def test_forced_configuration_arguments(gpu):
+    abi = Abi()
+    try:
+        L, n, p = abi.L, len(_configs(abi.L)), abi.alloc(64 * 64 * 4)
+        run = L.aar_gemm_f32_with_split_config
+        assert run(NN, 64, 64, 64, p, p, p, None, 0, n, 1, None) == -1
+        assert run(NN, 64, 64, 64, p, p, p, None, 0, -1, 1, None) == -1
+        assert run(NN, 64, 64, 64, p, p, p, None, 0, 0, 0, None) == -1
+        assert run(NN, 64, 64, 256, p, p, p, None, 0, 0, 2, None) == -2  # no workspace
+        assert run(NT, 1, 1, 1 << 22, p, p, p, None, 0, 0, 1, None) == -3  # 32-bit offsets within a tile
+    finally:
+        abi.free()

@@ -67,7 +67,7 @@ def _sentinel_words(abi, rows, cols):
 SHAPES = [
     (16384, 1536, 384, 384),  # GPT block (must be fused)
     (4096, 1536, 384, 384),
-    (4004, 1536, 384, 384),   # forward on the 32-row wave tiles of configuration 16, a 4-row last word
+    (4004, 1536, 384, 384),   # a 4-row last word
     (2048, 960, 384, 128),
     (1000, 200, 64, 96),      # M not a multiple of 32: a partial last word (forward only)
     (1024, 200, 64, 96),      # N not a multiple of the tile width
@@ -155,8 +155,8 @@ SPLIT_K = {NT: [(2048, 2048, 1920), (1280, 3000, 2304), (1025, 3072, 2560), (100
            NN: [(2304, 2304, 1920), (2304, 2304, 2560), (1920, 6144, 3072)]}
 
 
-@pytest.mark.parametrize("op,M,N,K", [(op, *s) for op in SPLIT_K for s in SPLIT_K[op]])
-def test_taken_where_k_might_be_split(gpu, op, M, N, K):
+def check_taken(op, M, N, K):
+    """The fused call of the layout takes aligned operands of the shape."""
     abi = Abi()
     L = abi.L
     _bind(L)
@@ -172,6 +172,11 @@ def test_taken_where_k_might_be_split(gpu, op, M, N, K):
             abi.check(L.aar_gemm_f32_mask_bits_colsum(NN, M, N, K, p, q, pbits, pc, None, None, 0, None))
     finally:
         abi.free()
+
+
+@pytest.mark.parametrize("op,M,N,K", [(op, *s) for op in SPLIT_K for s in SPLIT_K[op]])
+def test_taken_where_k_might_be_split(gpu, op, M, N, K):
+    check_taken(op, M, N, K)
     d, N2 = (K, 64) if op == NT else (64, K)
     test_bits_forward_and_masked_backward(gpu, M, N, d, N2)
 
