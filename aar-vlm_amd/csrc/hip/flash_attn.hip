@@ -1993,7 +1993,8 @@ int fa_fwd_query_block(int64_t bh, int64_t T, int64_t d, bool causal, bool vec, 
 // 0.83-1.10, 256 0.78-1.00, 320 0.71-0.92, 384 0.72-0.86, 777 0.62-0.74, 2048
 // 0.59-0.70; causal (d = 40; d = 64 takes the paired or split kernels below
 // about 2000 workgroups) T = 256 0.89-1.07, 384 0.81-1.06, 512 0.72-0.84, 777
-// 0.64-0.77, 2048 0.58-0.72: short rows do not pay for splitting Q and for the
+// 0.64-0.77, 2048 0.58-0.72 (not compared with the paired and split kernels where
+// those are planned): short rows do not pay for splitting Q and for the
 // longer first tile.  Head dims up to 32 stay: 0.8-1.2, with half the matrix
 // work per split element.
 bool fa_fwd_bf16x3(int64_t T, bool causal) { return T > (causal ? 384 : 256); }

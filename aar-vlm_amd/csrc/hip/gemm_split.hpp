@@ -24,7 +24,9 @@ struct GemmEpiArgs {
 // relative to a full CU.  Fitted to 3889 times (shape, layout, configuration,
 // split) on MI355X over 49 shapes from 100^3 and 64 x 64 x 4096 to 4096^3 and
 // 8192 x 8192 x 512, the GPT step's among them: the model's pick is 1.0 %
-// slower than the best on average and 12 % at most (20000 x 200 x 100).
+// slower than the best on average and 12 % at most (20000 x 200 x 100).  Its times
+// are for comparing plans: products that the chip's power bounds take 15-25 %
+// longer (4096^3 534 us by the model, 640-670 measured).
 // Measured and not built: 256 x 128 and 128 x 256 as four waves of 128 x 64 / 64
 // x 128 (one wave per SIMD: 4096^3 NN / NT / TN 650 / 642 / 675 us against
 // 641 / 625 / 646 for eight waves of 64 x 64; the GPT step's shapes 4-15 %

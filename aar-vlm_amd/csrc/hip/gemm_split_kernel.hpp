@@ -5,7 +5,7 @@
 //   TN  C[M,N] = A[K,M]^T . B[K,N]
 //
 // Bound by the matrix cores' power on large products: at 4096^3 the chip holds
-// 1.8 GHz with the unit 70 % busy, 1.3 PFLOP/s of bf16 products, where a large
+// 1.8 GHz with the unit 65 % busy, 1.24 PFLOP/s of bf16 products, where a large
 // plain bf16 product reaches 1.18 PFLOP/s at 4096^3 and 1.37 at 16384^3 on this
 // card.  So the work around it is kept small:
 //  * Each element is split once per workgroup, not once per wave: tiles go
